@@ -1978,14 +1978,34 @@ const void* cycle_table_device(const CycleTable& t, hipError_t* err) {
   return p;
 }
 
+// Steps of D positions for short cycles: a pass whose segments average at
+// most D positions computes no source positions past their ends (D = 8 over
+// 2-cycles of composed maps spent three quarters of its instructions there).
+template <typename Word, int D>
+void launch_cycle_short(const CycArgs& a, int variant, uint32_t blocks, hipStream_t stream) {
+  if (variant == 4)
+    hipLaunchKernelGGL((k_cycle<Word, D, 2>), dim3(blocks), dim3(256), 0, stream, a);
+  else if (variant == 5)
+    hipLaunchKernelGGL((k_cycle<Word, D, 3>), dim3(blocks), dim3(256), 0, stream, a);
+  else
+    hipLaunchKernelGGL((k_cycle<Word, D>), dim3(blocks), dim3(256), 0, stream, a);
+}
+
 template <typename Word>
-hipError_t launch_cycle_w(CycArgs a, int variant, hipStream_t stream) {
+hipError_t launch_cycle_w(CycArgs a, int variant, uint32_t mean, hipStream_t stream) {
   if (a.nslots) {
     const uint64_t words = a.B * a.nslots * (a.U / sizeof(Word));
     const uint64_t blocks = std::min<uint64_t>((words + 255) / 256, 256ull * 64);
     hipLaunchKernelGGL((k_cycle_save<Word>), dim3((uint32_t)blocks), dim3(256), 0, stream, a);
   }
   const uint64_t blocks = ((a.items << a.lane_log2) + 255) / 256;
+  if constexpr (sizeof(Word) == 16) {
+    if ((variant == 0 || variant == 4 || variant == 5) && mean && mean <= 4) {
+      if (mean <= 2) launch_cycle_short<Word, 2>(a, variant, (uint32_t)blocks, stream);
+      else launch_cycle_short<Word, 4>(a, variant, (uint32_t)blocks, stream);
+      return hipGetLastError();
+    }
+  }
   if (a.lane_log2 < 6 && variant >= 1 && variant <= 3)  // one item per wave only
     hipLaunchKernelGGL((k_cycle<Word, 8>), dim3((uint32_t)blocks), dim3(256), 0, stream, a);
   else if (variant == 1)
@@ -2439,12 +2459,13 @@ hipError_t launch_cycle(const Op& op, char* data, char* scratch, int64_t scratch
   // 256 MB last-level cache could hold, was 30 % slower with them
   if (variant == 0 && w == 16 && a.U >= 512) variant = 5;
   else if (variant == 0 && w == 16 && a.B * a.RCU >= (512ull << 20)) variant = 4;
+  const uint32_t mean = op.cyc->mean;
   switch (w) {
-    case 16: return launch_cycle_w<W16>(a, variant, stream);
-    case 8: return launch_cycle_w<uint64_t>(a, variant, stream);
-    case 4: return launch_cycle_w<uint32_t>(a, variant, stream);
-    case 2: return launch_cycle_w<uint16_t>(a, variant, stream);
-    default: return launch_cycle_w<uint8_t>(a, variant, stream);
+    case 16: return launch_cycle_w<W16>(a, variant, mean, stream);
+    case 8: return launch_cycle_w<uint64_t>(a, variant, mean, stream);
+    case 4: return launch_cycle_w<uint32_t>(a, variant, mean, stream);
+    case 2: return launch_cycle_w<uint16_t>(a, variant, mean, stream);
+    default: return launch_cycle_w<uint8_t>(a, variant, mean, stream);
   }
 }
 

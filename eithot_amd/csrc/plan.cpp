@@ -614,6 +614,24 @@ std::shared_ptr<CycleTable> choose_cycle_table(const std::vector<CycleMap>& maps
     lmax = lmax >= N ? N : lmax * 2;
     t = build_cycle_table_maps(maps, N, lmax);
   }
+  // Cells under 1 KiB share a wave, which runs until its longest segment
+  // ends: segments of short cycles are grouped by length in steps of 8 (the
+  // kernel's unrolled step), longest first, each group in its own order (a
+  // counting sort, so neighbouring starts stay neighbours).  A 207 MB pass
+  // of 128-byte cells with cycles of 1 to 60 positions: 126 -> 122 us.  Long
+  // cycles, cut into nearly equal segments, keep their order, which the
+  // grouping disturbs (4.5 GB, 128-byte cells: 2 % slower with it).
+  t->mean = t->mean_len();
+  if (U < 1024 && t->mean <= 32) {
+    constexpr uint32_t kGroups = 33;  // the last takes every length above 256
+    auto group = [](const CycleSeg& s) { return kGroups - 1 - std::min((s.len - 1) / 8, kGroups - 1); };
+    std::vector<size_t> at(kGroups + 1, 0);
+    for (const CycleSeg& s : t->segs) ++at[group(s) + 1];
+    for (uint32_t g = 0; g < kGroups; ++g) at[g + 1] += at[g];
+    std::vector<CycleSeg> sorted(t->segs.size());
+    for (const CycleSeg& s : t->segs) sorted[at[group(s)]++] = s;
+    t->segs.swap(sorted);
+  }
   return t;
 }
 

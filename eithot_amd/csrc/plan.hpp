@@ -99,6 +99,13 @@ struct CycleTable {
   std::vector<CycleMap> maps;
   std::vector<CycleSeg> segs;
   std::vector<uint32_t> slots;  // slot -> position whose old cell it holds
+  // positions per segment, rounded up: sizes the kernel's unrolled steps
+  uint32_t mean_len() const {
+    uint64_t n = 0;
+    for (const CycleSeg& s : segs) n += s.len;
+    return segs.empty() ? 0 : (uint32_t)((n + segs.size() - 1) / segs.size());
+  }
+  uint32_t mean = 0;  // mean_len(), set once the table is final
   int64_t bytes() const { return (int64_t)(segs.size() * sizeof(CycleSeg) + slots.size() * 4); }
   // device copies (segs then slots), one per device id, made by the launcher
   DeviceCopies dev;
