@@ -86,6 +86,18 @@ void batch_launch_free(BatchLaunch* L);
 int64_t batch_launch_items(const BatchLaunch* L);
 int batch_launch_count(const BatchLaunch* L);  // kernel launches per enqueue
 
+// The whole-permutation pass `p` over the tensor at `data` (whole.hip).  A
+// resident pass whose workgroups do not meet within `patience` ticks of the
+// 100 MHz clock sets *host_failed and leaves the tensor indeterminate.
+struct WholePass;
+struct WholeTurn {
+  uint32_t pass = 0;  // number of this resident pass on its device, from 1, never 0
+  uint64_t patience = 0;
+  uint32_t* host_failed = nullptr;
+};
+hipError_t launch_whole(const WholePass& p, char* data, const WholeTurn& turn, hipStream_t stream);
+hipError_t configure_whole(int64_t bytes);
+
 // Raise the dynamic-LDS limit of every pass kernel to `bytes` (once per device).
 hipError_t configure_kernels(int64_t bytes);
 

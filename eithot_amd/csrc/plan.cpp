@@ -943,8 +943,17 @@ static int64_t* tuning_field(Tuning& t, const char* key) {
   if (!strcmp(key, "hold_floor")) return &t.hold_floor;
   if (!strcmp(key, "cycle_u_depth")) return &t.cycle_u_depth;
   if (!strcmp(key, "min_groups")) return &t.min_groups;
+  if (!strcmp(key, "whole")) return &t.whole;
   return nullptr;
 }
+
+// the knobs that choose or shape the passes of a plan
+constexpr const char* kPassKnobs[] = {
+    "lds_target",     "tile_fp_target", "slice_min",       "stage_chunk",     "cycle_min_cell",
+    "fuse_max_block", "block_digits",   "block_pad",       "cycle_word_cost", "threads",
+    "threads_big",    "xcd_remap",      "cycle_variant",   "reorder",         "regroup",
+    "cycle_lmax",     "cycle_cell_pref", "segtile_threads", "lds_threads_auto", "segtile_nt",
+    "lower_mask",     "cycle_u_depth",  "min_groups"};
 
 int tuning_set(const char* key, int64_t value) {
   std::lock_guard<std::mutex> lk(g_tune_mu);
@@ -964,9 +973,12 @@ int tuning_set(const char* key, int64_t value) {
   if (f == &t.min_groups && (value < 1 || value > (1 << 20))) return EITHOT_ERR_INVALID;
   const bool flag = f == &t.regroup || f == &t.lds_threads_auto || f == &t.cycle_cell_pref ||
                     f == &t.cycle_word_cost || f == &t.block_digits || f == &t.block_pad ||
-                    f == &t.xcd_remap;
+                    f == &t.xcd_remap || f == &t.whole;
   if (flag && value > 1) return EITHOT_ERR_INVALID;
   *f = value;
+  Tuning def;
+  t.plain = true;
+  for (const char* k : kPassKnobs) t.plain = t.plain && *tuning_field(t, k) == *tuning_field(def, k);
   t.epoch = g_tune.epoch + 1;
   g_tune = t;
   return EITHOT_OK;
@@ -996,6 +1008,8 @@ void tuning_apply(const Tuning& t, DeviceProfile& prof) {
   prof.cycle_lmax = t.cycle_lmax;
   prof.cycle_cell_pref = t.cycle_cell_pref;
   prof.lower_mask = t.lower_mask;
+  // a caller who sets any knob of the passes asks for those passes
+  prof.whole = t.whole != 0 && t.plain;
 }
 
 void lower_transpose2d(int64_t B, int64_t R, int64_t C, int64_t U, uint64_t base, int stage,

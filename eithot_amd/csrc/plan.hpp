@@ -203,6 +203,7 @@ struct DeviceProfile {
   int64_t cycle_lmax = 0;         // > 0: cycle segments of at most this many positions
   int64_t cycle_cell_pref = 0;    // 1: cycle passes of larger cells cost less
   int64_t lower_mask = LOWER_ALL; // lowering options the planner may use
+  int whole = 1;                  // one whole-permutation pass where it fits (whole.hpp)
   int cycle_shift = 1;            // cycle passes of narrow cells run the shifted 16-byte
                                   // kernel (0: word by word, as in batched launches)
   double staged_mult = 1.0;       // planner-internal: weight of staged passes in the search
@@ -235,12 +236,16 @@ struct Tuning {
   int64_t hold_floor = 64ll << 20;  // device bytes the library may keep whatever alpha allows
   int64_t cycle_u_depth = 4;        // positions in flight per item of the shifted cycle kernel (4, 6, 8)
   int64_t min_groups = 1024;        // workgroups a single-launch pass spreads its footprints over
+  int64_t whole = 1;                // whole-permutation passes (whole.hpp) where they fit
+  bool plain = true;   // every knob of the passes has its default value
   uint64_t epoch = 0;  // bumped on every change (plan caches key on it)
 };
 Tuning tuning_get();
 int tuning_set(const char* key, int64_t value);  // 0 or EITHOT_ERR_INVALID
 int tuning_value(const char* key, int64_t* value);
 void tuning_apply(const Tuning& t, DeviceProfile& prof);
+
+struct WholePass;  // whole.hpp
 
 struct Plan {
   std::vector<Stage> stages;
@@ -261,6 +266,9 @@ struct Plan {
   // segmented tile's block order), created on its first run; the runtime
   // serialises access to it.
   mutable std::shared_ptr<void> launch_state;
+  // One pass that does the work of all of `ops` where the tensor allows it;
+  // the runtime prefers it (null: none).
+  std::shared_ptr<const WholePass> whole;
 };
 
 // Full plan.  perm1 is 1-based.  alpha bounds the scratch (scratch <= alpha *

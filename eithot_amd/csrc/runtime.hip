@@ -66,6 +66,7 @@ Device* device_ctx(int* err) {
     d->prof.lds_max = std::min<int64_t>(lds, 160 * 1024);
     d->prof.lds_target = std::min<int64_t>(64 * 1024, d->prof.lds_max);
     hipError_t e = configure_kernels(d->prof.lds_max);
+    if (e == hipSuccess) e = configure_whole(d->prof.lds_max);
     if (e != hipSuccess) {
       // fall back to the per-block limit the runtime reports
       d->prof.lds_max = (int64_t)prop.sharedMemPerBlock;
@@ -111,6 +112,21 @@ std::string plan_key(const int64_t* dims, const int* perm1, int rank, size_t ele
   return k.str();
 }
 
+// Whether the only pass of a plan is one that a whole-permutation pass beats
+// on tensors of up to 64 MiB: a staged pass; a cycle pass that also saves
+// boundary cells, or moves cells of narrow words (0.6 MB: 17 -> 10 us, 15 MB:
+// 42 -> 23 us; without either, 0.9 MB: 9 us, 12 in one pass); an LDS pass of
+// few workgroups with 40 KiB and more each (77 KB: 17 -> 9.5 us; with 16 KiB:
+// 8.3 us, 10.3 in one pass).
+static bool only_pass_weak(const Plan& p) {
+  if (p.ops.size() != 1 || p.tensor_bytes > (64ull << 20)) return false;
+  const Op& o = p.ops[0];
+  if (o.staged) return true;
+  if (o.kind == OP_CYCLE) return o.cyc && (!o.cyc->slots.empty() || o.U % 16);
+  const int64_t n = o.kind == OP_BLOCK || o.kind == OP_SEGTILE ? o.B : o.num_footprints();
+  return n < 64 && p.tensor_bytes / (uint64_t)n >= 40 * 1024;
+}
+
 PlanPtr Device::plan_for(const int64_t* dims, const int* perm1, int rank, size_t elem, int n_sub,
                          double alpha, int* rc) {
   const DeviceProfile pr = profile();
@@ -127,6 +143,11 @@ PlanPtr Device::plan_for(const int64_t* dims, const int* perm1, int rank, size_t
   auto p = std::make_shared<Plan>();
   *rc = make_plan(dims, perm1, rank, elem, n_sub, alpha, pr, pr.reorder, *p);
   if (*rc != EITHOT_OK) return nullptr;
+  if (pr.whole) {
+    const WholePass w = plan_whole(dims, perm1, rank, elem, pr.cus, pr.lds_max, (int)p->ops.size(),
+                                   only_pass_weak(*p));
+    if (w.mode != WHOLE_NONE) p->whole = std::make_shared<const WholePass>(w);
+  }
   std::vector<PlanPtr> evicted;  // destroyed after the lock is released
   PlanPtr out;
   {
@@ -173,9 +194,13 @@ void Device::trim_locked(int64_t budget, const Plan* keep) {
   }
 }
 
+bool stream_captured(hipStream_t stream);
+
 int Device::reserve_arena_locked(int64_t bytes, hipStream_t stream) {
   if (bytes <= 0) return EITHOT_OK;
-  if (arena_ready) {  // earlier async users of the arena must finish first
+  // earlier async users of the arena must finish first (a captured call has
+  // nothing to wait for yet: its replays come later)
+  if (arena_ready && !stream_captured(stream)) {
     if (hipStreamWaitEvent(stream, arena_ready, 0) != hipSuccess)
       return fail(EITHOT_ERR_DEVICE, "hipStreamWaitEvent failed");
   }
@@ -198,11 +223,88 @@ int Device::reserve_arena_locked(int64_t bytes, hipStream_t stream) {
 }
 
 int Device::release_arena_after_locked(hipStream_t stream) {
+  // an event recorded into a capture would order nothing, and could not be
+  // waited for by eager calls
+  if (stream_captured(stream)) return EITHOT_OK;
   if (!arena_ready && hipEventCreateWithFlags(&arena_ready, hipEventDisableTiming) != hipSuccess)
     return fail(EITHOT_ERR_DEVICE, "hipEventCreate failed");
   if (hipEventRecord(arena_ready, stream) != hipSuccess)
     return fail(EITHOT_ERR_DEVICE, "hipEventRecord failed");
   return EITHOT_OK;
+}
+
+// ticks of the 100 MHz clock that a resident pass waits for its workgroups
+// (20 s; they meet within microseconds unless other processes hold the chip)
+constexpr uint64_t kWholePatience = 2000000000ull;
+
+bool stream_captured(hipStream_t stream) {
+  if (!stream) return false;  // the null stream cannot be
+  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(stream, &cap) != hipSuccess) {
+    (void)hipGetLastError();
+    return true;  // unknown: treat as captured
+  }
+  return cap != hipStreamCaptureStatusNone;
+}
+
+bool Device::takes_whole_locked(const Plan& plan, hipStream_t stream) {
+  if (!plan.whole) return false;
+  if (plan.whole->mode == WHOLE_ORBIT) return true;
+  if (whole_off || stream_captured(stream)) return false;
+  if (!whole_failed) {
+    if (hipHostMalloc((void**)&whole_failed, sizeof(uint32_t), hipHostMallocDefault) != hipSuccess) {
+      (void)hipGetLastError();
+      whole_failed = nullptr;
+      return false;
+    }
+    *whole_failed = 0;
+  }
+  if (!whole_ready && hipEventCreateWithFlags(&whole_ready, hipEventDisableTiming) != hipSuccess) {
+    (void)hipGetLastError();
+    whole_ready = nullptr;
+    return false;
+  }
+  return true;
+}
+
+int Device::launch_whole_locked(const Plan& plan, char* data, hipStream_t stream) {
+  const bool chain = plan.whole->mode == WHOLE_RESIDENT;
+  // a plan called once can be captured into a graph, where it runs its
+  // ordinary passes: their tables are uploaded all the same
+  if (chain && plan.table_bytes > 0 && plan.device_table_bytes(id) < plan.table_bytes)
+    for (const Op& o : plan.ops)
+      if (prepare_op(o) != hipSuccess) return fail(EITHOT_ERR_DEVICE, "uploading a pass table failed");
+  // Passes on the null stream follow each other by themselves; the event is
+  // recorded behind them only when a call on another stream needs it (the
+  // null stream outlives every call, other streams may not).
+  if (chain && (stream || whole_elsewhere)) {
+    if (!whole_elsewhere && hipEventRecord(whole_ready, nullptr) != hipSuccess)
+      return fail(EITHOT_ERR_DEVICE, "hipEventRecord failed");
+    if (hipStreamWaitEvent(stream, whole_ready, 0) != hipSuccess)
+      return fail(EITHOT_ERR_DEVICE, "hipStreamWaitEvent failed");
+  }
+  WholeTurn& t = whole_turn;
+  if (chain) {
+    if (++t.pass == 0) ++t.pass;
+    t.patience = kWholePatience;
+    t.host_failed = whole_failed;
+  }
+  const hipError_t e = launch_whole(*plan.whole, data, t, stream);
+  if (e != hipSuccess)
+    return fail(EITHOT_ERR_DEVICE, "whole pass launch failed: %s", hipGetErrorString(e));
+  if (chain) whole_elsewhere = stream != nullptr;
+  if (chain && stream && hipEventRecord(whole_ready, stream) != hipSuccess)
+    return fail(EITHOT_ERR_DEVICE, "hipEventRecord failed");
+  return EITHOT_OK;
+}
+
+int Device::whole_status() {
+  std::lock_guard<std::mutex> lk(enqueue_mu);
+  if (whole_off || !whole_failed || !*(volatile uint32_t*)whole_failed) return EITHOT_OK;
+  whole_off = true;
+  return fail(EITHOT_ERR_DEVICE,
+              "a resident pass gave up waiting for its workgroups; the tensors of calls since the "
+              "last synchronisation are indeterminate");
 }
 
 // Timing events of this thread on each device, reused from call to call
@@ -325,12 +427,20 @@ int run_plan(Device* d, const Plan& plan, char* data, char* scratch, int64_t scr
     }
   }
   int rc = EITHOT_OK;
+  const bool whole = d->takes_whole_locked(plan, stream);
+  const size_t npass = whole ? 1 : plan.ops.size();
+  if (whole) {
+    rc = d->launch_whole_locked(plan, data, stream);
+    if (rc == EITHOT_OK && times && hipEventRecord(ev[1], stream) != hipSuccess)
+      rc = fail(EITHOT_ERR_DEVICE, "pass timing event failed");
+    if (times) ev.resize(2);
+  }
   LaunchCfg cfg = d->launch_cfg();
   if (min_groups_cap > 0) cfg.min_groups = std::min(cfg.min_groups, min_groups_cap);
   std::vector<int> remap;
   std::vector<std::pair<hipEvent_t, hipEvent_t>> rec;
-  seg_orders(plan, cfg.xcd_remap, stream, remap, rec);
-  for (size_t i = 0; i < plan.ops.size(); ++i) {
+  if (!whole) seg_orders(plan, cfg.xcd_remap, stream, remap, rec);
+  for (size_t i = 0; !whole && i < plan.ops.size(); ++i) {
     LaunchCfg c = cfg;
     c.xcd_remap = remap[i];
     if (rec[i].first && hipEventRecord(rec[i].first, stream) != hipSuccess) (void)hipGetLastError();
@@ -351,7 +461,7 @@ int run_plan(Device* d, const Plan& plan, char* data, char* scratch, int64_t scr
     if (rc == EITHOT_OK) {
       if (hipEventSynchronize(ev.back()) != hipSuccess)
         return fail(EITHOT_ERR_DEVICE, "pass timing synchronisation failed");
-      for (size_t i = 0; i < plan.ops.size(); ++i) {
+      for (size_t i = 0; i < npass; ++i) {
         float ms = 0;
         if (hipEventElapsedTime(&ms, ev[i], ev[i + 1]) != hipSuccess) {
           times->clear();
@@ -400,18 +510,23 @@ static int transpose_impl(void* dev, const int64_t* dims, const int* perm, int o
     if (!g_err.size()) fail(rc, "planning failed (%d)", rc);
     return rc;
   }
+  if ((rc = d->whole_status())) return rc;
   {
     std::lock_guard<std::mutex> lk(d->enqueue_mu);
+    const bool whole = d->takes_whole_locked(*plan, stream);
     // the library's device bytes stay within alpha of this tensor, or this
     // plan's own need when one footprint exceeds it, or the holding floor
     // (which spares calls on small tensors from evicting and re-uploading
     // the tables of the others)
-    const int64_t own = plan->scratch_bytes + plan->table_bytes;
+    // a resident pass needs no extra memory, but keeps what a captured call of
+    // its plan will use
+    const bool keeps = !whole || plan->whole->mode == WHOLE_RESIDENT;
+    const int64_t own = keeps ? plan->scratch_bytes + plan->table_bytes : 0;
     const int64_t budget = std::max<int64_t>(
         std::max<int64_t>((int64_t)(alpha * (double)plan->tensor_bytes), own),
         tuning_get().hold_floor);
-    d->trim_locked(budget, plan.get());
-    if (plan->scratch_bytes > 0) {
+    d->trim_locked(budget, keeps ? plan.get() : nullptr);
+    if (whole ? keeps && d->arena_bytes < plan->scratch_bytes : plan->scratch_bytes > 0) {
       rc = d->reserve_arena_locked(plan->scratch_bytes, stream);
       if (rc) return rc;
     }
@@ -419,7 +534,7 @@ static int transpose_impl(void* dev, const int64_t* dims, const int* perm, int o
     TableAccount acct(&d->cached_tables);
     rc = run_plan(d, *plan, (char*)dev, d->arena, plan->scratch_bytes, stream, times);
     if (rc) return rc;
-    if (plan->scratch_bytes > 0) {
+    if (!whole && plan->scratch_bytes > 0) {
       rc = d->release_arena_after_locked(stream);
       if (rc) return rc;
     }
@@ -429,6 +544,7 @@ static int transpose_impl(void* dev, const int64_t* dims, const int* perm, int o
     hipError_t e = hipStreamSynchronize(stream);
     if (e == hipSuccess) e = hipGetLastError();
     if (e != hipSuccess) return fail(EITHOT_ERR_DEVICE, "device error: %s", hipGetErrorString(e));
+    if ((rc = d->whole_status())) return rc;
   }
   return EITHOT_OK;
 }

@@ -12,6 +12,7 @@
 #include "kernels.hpp"
 #include "plan.hpp"
 #include "plan_cache.hpp"
+#include "whole.hpp"
 
 namespace eithot {
 
@@ -34,6 +35,15 @@ struct Device {
   char* arena = nullptr;             // scratch for staged passes and cycle boundaries
   int64_t arena_bytes = 0;
   hipEvent_t arena_ready = nullptr;  // recorded after the last pass that used the arena
+  // Resident whole-permutation passes share the chip with no other of their
+  // kind (whole.hip): each waits, on the device, for the one before.  Once
+  // one has given up waiting (*whole_failed, written by the kernel) the
+  // device runs ordinary passes only.  All under enqueue_mu.
+  hipEvent_t whole_ready = nullptr;
+  bool whole_elsewhere = false;      // the last one ran on a stream other than the null stream
+  uint32_t* whole_failed = nullptr;  // pinned host memory
+  bool whole_off = false;
+  WholeTurn whole_turn;
   // device bytes of the pass tables uploaded for plans of this cache (and
   // not yet freed; an evicted plan a request still holds counts until freed)
   std::atomic<int64_t> cached_tables{0};
@@ -59,6 +69,14 @@ struct Device {
   // user on `stream`.
   int reserve_arena_locked(int64_t bytes, hipStream_t stream);
   int release_arena_after_locked(hipStream_t stream);
+  // With enqueue_mu held: whether a call of `plan` on `stream` runs its
+  // whole-permutation pass, and the launch of it.  Resident passes are left
+  // out of stream captures (a replay could not be chained).
+  bool takes_whole_locked(const Plan& plan, hipStream_t stream);
+  int launch_whole_locked(const Plan& plan, char* data, hipStream_t stream);
+  // Reports (once) that a resident pass gave up: its tensor's contents are
+  // indeterminate.  EITHOT_OK otherwise.
+  int whole_status();
   // Device bytes the library holds for plain transposes on this device.
   int64_t held_bytes();
 };

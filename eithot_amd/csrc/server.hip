@@ -117,7 +117,7 @@ struct eithot_server {
         continue;
       }
       r->latency_ms = ns / 1e6;
-      r->status = 2;
+      r->status = r->plan->whole && dev->whole_status() ? EITHOT_ERR_DEVICE : 2;
       pool.release(r->off, r->bytes);
       --stream_load[r->stream];
       free_events.push_back(r->done_ev);

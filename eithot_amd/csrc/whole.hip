@@ -1,0 +1,408 @@
+// gfx950 kernels of the whole-permutation passes (whole.hpp).
+#include <hip/hip_runtime.h>
+
+#include "kernels.hpp"
+#include "whole.hpp"
+
+namespace eithot {
+namespace {
+
+typedef uint32_t V16 __attribute__((ext_vector_type(4)));
+// global accesses of 16 bytes at any address (runs start where the tensor's
+// lengths put them); the hardware splits them at line boundaries
+typedef uint32_t V16u __attribute__((ext_vector_type(4), aligned(1)));
+
+template <int WL>
+struct ElemOf;
+template <>
+struct ElemOf<0> {
+  using T = uint8_t;
+};
+template <>
+struct ElemOf<1> {
+  using T = uint16_t;
+};
+template <>
+struct ElemOf<2> {
+  using T = uint32_t;
+};
+template <>
+struct ElemOf<3> {
+  using T = uint64_t;
+};
+template <>
+struct ElemOf<4> {
+  using T = V16;
+};
+// an element at any global address
+template <int WL>
+struct Loose {
+  typename ElemOf<WL>::T v;
+} __attribute__((packed));
+
+template <int WL>
+union Chunk {
+  typename ElemOf<WL>::T e[16 >> WL];
+  V16 v;
+};
+
+// 16 bytes to LDS at a multiple of max(4, element) bytes
+template <int WL>
+__device__ __forceinline__ void put_chunk(unsigned char* p, const V16& v) {
+  if constexpr (WL == 4) {
+    *reinterpret_cast<V16*>(p) = v;
+  } else if constexpr (WL == 3) {
+    reinterpret_cast<uint64_t*>(p)[0] = (uint64_t)v[0] | ((uint64_t)v[1] << 32);
+    reinterpret_cast<uint64_t*>(p)[1] = (uint64_t)v[2] | ((uint64_t)v[3] << 32);
+  } else {
+    uint32_t* q = reinterpret_cast<uint32_t*>(p);
+    q[0] = v[0];
+    q[1] = v[1];
+    q[2] = v[2];
+    q[3] = v[3];
+  }
+}
+
+// LDS areas of a workgroup (whole.hpp)
+struct Areas {
+  uint32_t* in;    // input runs: offsets from the tile's first element
+  uint2* out;      // output runs: the same, and their LDS offsets
+  uint32_t* otab;  // LDS offsets of an output run's elements
+  unsigned char* tile;
+};
+__device__ __forceinline__ Areas areas(const WholeGeom& g, unsigned char* lds) {
+  Areas a;
+  a.in = reinterpret_cast<uint32_t*>(lds + kWholeCtl);
+  a.out = reinterpret_cast<uint2*>(lds + kWholeCtl + whole_in_bytes(g));
+  a.otab = reinterpret_cast<uint32_t*>(lds + kWholeCtl + whole_in_bytes(g) + whole_out_bytes(g));
+  a.tile = reinterpret_cast<unsigned char*>(a.otab) + whole_otab_bytes(g);
+  return a;
+}
+
+constexpr uint32_t kNoRun = ~0u;
+
+template <int ND>
+__device__ __forceinline__ void list_in(const WholeGeom& g, const WholeTile& x, const Areas& a) {
+  for (uint32_t e = threadIdx.x; e < g.nin; e += blockDim.x) {
+    uint32_t off;
+    const bool ok = whole_in_run<ND>(g, x, e, &off);
+    a.in[e] = ok ? off : kNoRun;
+  }
+}
+template <int ND>
+__device__ __forceinline__ void list_out(const WholeGeom& g, const WholeTile& x, const Areas& a) {
+  for (uint32_t e = threadIdx.x; e < g.nout; e += blockDim.x) {
+    uint32_t off, l;
+    const bool ok = whole_out_run<ND>(g, x, e, &off, &l);
+    a.out[e] = make_uint2(ok ? off : kNoRun, l);
+  }
+}
+template <bool MULTI, int ND>
+__device__ __forceinline__ void list_elems(const WholeGeom& g, const Areas& a) {
+  if (MULTI)
+    for (uint32_t e = threadIdx.x; e < g.len_out; e += blockDim.x) a.otab[e] = whole_elem<ND>(g, e);
+}
+
+// A thread's walk over the 16-byte chunks t = threadIdx.x + i * blockDim.x of
+// a tile's runs, `per` to a run: the run and the chunk within it step by
+// constants, so only the first takes a division.
+struct Walk {
+  uint32_t rho, c, drho, dc, per;
+  __device__ __forceinline__ Walk(const FD32& f) {
+    per = f.d;
+    rho = f.div(threadIdx.x);
+    c = threadIdx.x - rho * per;
+    drho = f.div(blockDim.x);
+    dc = blockDim.x - drho * per;
+  }
+  __device__ __forceinline__ void step() {
+    c += dc;
+    rho += drho;
+    const bool wrap = c >= per;
+    c -= wrap ? per : 0;
+    rho += wrap ? 1 : 0;
+  }
+};
+
+// Issues the loads of up to 8 chunks of the tile's input runs (src: the
+// tile's first element, room: the tensor's bytes from there on); at[u] is
+// chunk u's place in LDS, kNoRun for none.  Bytes read past a run's end are
+// never used; a chunk that would leave the tensor (whose size is at least 16
+// bytes) reads its last 16 bytes and shifts them down.
+__device__ __forceinline__ void get_chunks(const WholeGeom& g, const char* src, uint64_t room,
+                                           uint32_t run_bytes, const Areas& a, Walk& k, V16 (&v)[8],
+                                           uint32_t (&at)[8]) {
+  const uint32_t lim = room < kNoRun ? (uint32_t)room : kNoRun;
+#pragma unroll
+  for (int u = 0; u < 8; ++u) {
+    at[u] = kNoRun;
+    if (k.rho < g.nin) {
+      const uint32_t run = a.in[k.rho], c = k.c * 16;
+      if (run != kNoRun && c < run_bytes) {
+        at[u] = whole_row(g, k.rho) + c;
+        const uint32_t off = run + c;
+        if (off + 16 <= lim) {
+          v[u] = *reinterpret_cast<const V16u*>(src + off);
+        } else {
+          const V16 e = *reinterpret_cast<const V16u*>(src + (int64_t)room - 16);
+          const uint32_t s = (uint32_t)((uint64_t)off + 16 - room) * 8;
+          const uint64_t lo = (uint64_t)e[0] | ((uint64_t)e[1] << 32);
+          const uint64_t hi = (uint64_t)e[2] | ((uint64_t)e[3] << 32);
+          const uint64_t l = s < 64 ? (lo >> s) | (hi << 1 << (63 - s)) : hi >> (s - 64);
+          const uint64_t h = s < 64 ? hi >> s : 0;
+          v[u] = V16{(uint32_t)l, (uint32_t)(l >> 32), (uint32_t)h, (uint32_t)(h >> 32)};
+        }
+      }
+    }
+    k.step();
+  }
+}
+template <int WL>
+__device__ __forceinline__ void put_chunks(const Areas& a, const V16 (&v)[8], const uint32_t (&at)[8]) {
+#pragma unroll
+  for (int u = 0; u < 8; ++u)
+    if (at[u] != kNoRun) put_chunk<WL>(a.tile + at[u], v[u]);
+}
+
+// Stores the tile along its output runs (dst: its first element's place): 16
+// bytes per thread gathered from LDS element by element; a run's last store
+// is moved back to end with the run (its first elements are stored twice,
+// with the same values).
+template <int WL, bool MULTI, int ND>
+__device__ __forceinline__ void tile_store(const WholeGeom& g, const WholeTile& x, char* dst,
+                                           const Areas& a) {
+  using E = typename ElemOf<WL>::T;
+  constexpr uint32_t V = 16u >> WL;
+  const uint32_t len = whole_len_out<ND>(g, x);
+  Walk k(g.fcout);
+  for (; k.rho < g.nout; k.step()) {
+    const uint2 run = a.out[k.rho];
+    uint32_t p = k.c * V;
+    if (run.x == kNoRun || p >= len) continue;
+    const unsigned char* l = a.tile + run.y;
+    // runs over one dim: V elements from a multiple of V (or any place
+    // without the group padding) lie a constant step apart
+    const bool tail = p + V > len;
+    if (len >= V && !(tail && !MULTI && g.g2)) {
+      if (tail) p = len - V;
+      Chunk<WL> q;
+      if constexpr (MULTI) {
+#pragma unroll
+        for (uint32_t e = 0; e < V; ++e) q.e[e] = *reinterpret_cast<const E*>(l + a.otab[p + e]);
+      } else {
+        const unsigned char* s = l + whole_elem1(g, p);
+#pragma unroll
+        for (uint32_t e = 0; e < V; ++e) q.e[e] = *reinterpret_cast<const E*>(s + e * g.ols[0]);
+      }
+      *reinterpret_cast<V16u*>(dst + (run.x + (p << WL))) = q.v;
+    } else {
+      for (; p < len; ++p)
+        reinterpret_cast<Loose<WL>*>(dst + (run.x + (p << WL)))->v =
+            *reinterpret_cast<const E*>(l + (MULTI ? a.otab[p] : whole_elem1(g, p)));
+    }
+  }
+}
+
+// ---------------------------------------------------------------------------
+// resident form
+// ---------------------------------------------------------------------------
+// Words in which a device's resident passes count the workgroups that have
+// loaded their tiles: 16 counters per region (each on a line of its own: one
+// address takes about 30 ns per addition) and a root that the last workgroup
+// of each adds to, all zero between passes, and the number of the last pass
+// in which the region was complete.
+constexpr uint32_t kSubs = 16;
+struct WholeCtl {
+  uint32_t failed, pad[31];
+  uint32_t open[kWholeRegions];
+  uint32_t root[kWholeRegions];
+  uint32_t sub[kSubs][kWholeRegions];
+};
+__device__ WholeCtl g_ctl;
+
+__device__ __forceinline__ uint32_t ctl_add(uint32_t* p, uint32_t v) {
+  return __hip_atomic_fetch_add(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ uint32_t ctl_get(uint32_t* p) {
+  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ void ctl_set(uint32_t* p, uint32_t v) {
+  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// Counts workgroup t of the n of region b; true for the last one.
+__device__ __forceinline__ bool ctl_arrive(uint32_t b, uint32_t t, uint32_t n) {
+  const uint32_t subs = n <= kSubs ? 1 : kSubs;
+  const uint32_t j = t % subs, members = (n - j + subs - 1) / subs;
+  if (ctl_add(&g_ctl.sub[j][b], 1) != members - 1) return false;
+  ctl_set(&g_ctl.sub[j][b], 0);
+  if (subs == 1) return true;
+  if (ctl_add(&g_ctl.root[b], 1) != subs - 1) return false;
+  ctl_set(&g_ctl.root[b], 0);
+  return true;
+}
+
+// One tile per workgroup.  The tiles of a region have consecutive block
+// indices, and workgroups start in that order on each XCD, so those of the
+// earliest unfinished region all run as soon as as many as it has tiles are
+// resident, which the planner keeps to half of the chip's room; they wait
+// for nobody else.  Launches of this kernel on one device follow each other
+// (the runtime chains them), so no two share that room.  No data passes
+// between workgroups: the counters only order a region's loads, which are
+// complete once in LDS, before its stores, so they need no cache flush.  The
+// wait is bounded all the same: after `patience` ticks of the 100 MHz clock
+// a workgroup reports a failure and leaves without storing, and so do those
+// after it.
+template <int WL, bool MULTI, int ND>
+__global__ __launch_bounds__(1024) void k_resident(WholeGeom g, char* data, uint32_t pass,
+                                                   uint64_t patience, uint32_t* host_failed) {
+  extern __shared__ __align__(16) unsigned char lds[];
+  uint32_t* ctl = reinterpret_cast<uint32_t*>(lds);
+  const uint32_t b = g.ftiles.div(blockIdx.x), t = blockIdx.x - b * g.tiles;
+  const WholeTile x = whole_tile<ND>(g, whole_nth(g, t));
+  const uint64_t region = (uint64_t)b * g.region;
+  const Areas a = areas(g, lds);
+  list_in<ND>(g, x, a);
+  list_out<ND>(g, x, a);
+  list_elems<MULTI, ND>(g, a);
+  __syncthreads();
+  const uint32_t run_bytes = whole_len_in<ND>(g, x) << WL;
+  for (Walk k(g.fcin); k.rho < g.nin;) {
+    V16 v[8];
+    uint32_t at[8];
+    get_chunks(g, data + region + x.in, g.B * g.region - region - x.in, run_bytes, a, k, v, at);
+    put_chunks<WL>(a, v, at);
+  }
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    uint32_t ok = 1;
+    if (ctl_arrive(b, t, g.tiles)) {
+      ctl_set(&g_ctl.open[b], pass);
+    } else {
+      const uint64_t t0 = __builtin_amdgcn_s_memrealtime();
+      for (;;) {
+        const uint32_t failed = ctl_get(&g_ctl.failed), now = ctl_get(&g_ctl.open[b]);
+        if (!failed && now == pass) break;
+        if (failed || __builtin_amdgcn_s_memrealtime() - t0 > patience) {
+          ctl_set(&g_ctl.failed, 1);
+          __hip_atomic_store(host_failed, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+          ok = 0;
+          break;
+        }
+        __builtin_amdgcn_s_sleep(1);
+      }
+    }
+    ctl[0] = ok;
+  }
+  __syncthreads();
+  if (ctl[0]) tile_store<WL, MULTI, ND>(g, x, data + region + x.out, a);
+}
+
+// ---------------------------------------------------------------------------
+// orbit form
+// ---------------------------------------------------------------------------
+// One cycle of tiles per workgroup: its tile with the lowest index leads,
+// the workgroups of the others leave.  The tile whose place the transposed
+// one takes is loaded into registers ahead of it and goes to LDS after it.
+template <int WL, bool MULTI, int ND>
+__global__ __launch_bounds__(512) void k_orbit(WholeGeom g, char* data) {
+  extern __shared__ __align__(16) unsigned char lds[];
+  const uint32_t b = g.ftiles.div(blockIdx.x);
+  const uint32_t first = whole_nth(g, blockIdx.x - b * g.tiles);
+  WholeTile x = whole_tile<ND>(g, first);
+  for (uint32_t q = x.next; q != first; q = whole_tile<ND>(g, q).next)
+    if (q < first) return;
+  char* base = data + (uint64_t)b * g.region;
+  const uint64_t room = (g.B - b) * g.region;
+  const Areas a = areas(g, lds);
+  list_in<ND>(g, x, a);
+  list_elems<MULTI, ND>(g, a);
+  __syncthreads();
+  V16 v[8];
+  uint32_t at[8];
+  Walk k(g.fcin);
+  get_chunks(g, base + x.in, room - x.in, whole_len_in<ND>(g, x) << WL, a, k, v, at);
+  for (;;) {
+    const bool more = x.next != first;
+    WholeTile y = x;
+    V16 nv[8];
+    uint32_t nat[8];
+    if (more) {
+      y = whole_tile<ND>(g, x.next);
+      __syncthreads();  // the list of x's input runs has been read
+      list_in<ND>(g, y, a);
+      __syncthreads();
+      Walk ky(g.fcin);
+      get_chunks(g, base + y.in, room - y.in, whole_len_in<ND>(g, y) << WL, a, ky, nv, nat);
+    }
+    list_out<ND>(g, x, a);
+    put_chunks<WL>(a, v, at);
+    __builtin_amdgcn_s_waitcnt(0);  // y is read before x is stored over it
+    __syncthreads();
+    tile_store<WL, MULTI, ND>(g, x, base + x.out, a);
+    if (!more) break;
+    __syncthreads();
+    x = y;
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+      v[u] = nv[u];
+      at[u] = nat[u];
+    }
+  }
+}
+
+template <int WL, bool MULTI, int ND>
+hipError_t launch_i(const WholePass& p, char* data, const WholeTurn& turn,
+                    hipStream_t st) {
+  const dim3 grid((uint32_t)(p.g.tiles * p.g.B)), block(p.threads);
+  if (p.mode == WHOLE_ORBIT)
+    hipLaunchKernelGGL((k_orbit<WL, MULTI, ND>), grid, block, (size_t)p.lds, st, p.g, data);
+  else
+    hipLaunchKernelGGL((k_resident<WL, MULTI, ND>), grid, block, (size_t)p.lds, st, p.g, data, turn.pass,
+                       turn.patience, turn.host_failed);
+  return hipGetLastError();
+}
+template <int WL>
+hipError_t launch_w(const WholePass& p, char* data, const WholeTurn& turn,
+                    hipStream_t st) {
+  const bool multi = p.g.jout > 1;
+  if (p.g.r <= 4)
+    return multi ? launch_i<WL, true, 4>(p, data, turn, st)
+                 : launch_i<WL, false, 4>(p, data, turn, st);
+  return multi ? launch_i<WL, true, kWholeDims>(p, data, turn, st)
+               : launch_i<WL, false, kWholeDims>(p, data, turn, st);
+}
+template <int WL>
+void configure_w(int64_t bytes, hipError_t& e) {
+  for (const void* fn : {(const void*)k_resident<WL, false, 4>, (const void*)k_resident<WL, true, 4>,
+                         (const void*)k_resident<WL, false, kWholeDims>,
+                         (const void*)k_resident<WL, true, kWholeDims>}) {
+    const hipError_t r = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
+    if (r != hipSuccess) e = r;
+  }
+}
+
+}  // namespace
+
+hipError_t launch_whole(const WholePass& p, char* data, const WholeTurn& turn,
+                        hipStream_t st) {
+  switch (p.g.w) {
+    case 16: return launch_w<4>(p, data, turn, st);
+    case 8: return launch_w<3>(p, data, turn, st);
+    case 4: return launch_w<2>(p, data, turn, st);
+    case 2: return launch_w<1>(p, data, turn, st);
+    default: return launch_w<0>(p, data, turn, st);
+  }
+}
+
+hipError_t configure_whole(int64_t bytes) {
+  hipError_t e = hipSuccess;
+  configure_w<0>(bytes, e);
+  configure_w<1>(bytes, e);
+  configure_w<2>(bytes, e);
+  configure_w<3>(bytes, e);
+  configure_w<4>(bytes, e);
+  return e;
+}
+
+}  // namespace eithot

@@ -149,6 +149,7 @@ typedef struct {
 } eithot_op_desc;
 
 /* Fills up to max_ops pass descriptors of the plan for the gfx950 profile
+ * (a call that the "whole" knob lets run in one pass does the same work in it)
  * (lds_max bytes of LDS per workgroup; <= 0 selects 160 KiB) and returns
  * the pass count; *scratch_bytes receives the plan's extra device memory
  * (scratch plus the cycle tables of its cycle-following passes). */
@@ -241,6 +242,12 @@ int eithot_plan_segments(const int64_t* dims, const int* perm, int order, size_t
  *                    round-robin) between timing events and later calls
  *                    keep the faster (not under graph capture); 0 forces
  *                    round-robin
+ *   "whole"          transpose in one pass that reads and writes every byte
+ *                    once, where the tensor allows it (lengths that read the
+ *                    same in input and output order, or regions that the
+ *                    chip's LDS holds whole), instead of the plan's passes (1;
+ *                    0: never).  Off while any knob of the passes differs
+ *                    from its default
  *   "hold_floor"     device bytes (arena and pass tables) the library may keep
  *                    after a call even when alpha * tensor bytes is smaller
  *                    (64 MiB; 0: alpha alone bounds them)
@@ -255,7 +262,8 @@ int eithot_get_tuning(const char* key, int64_t* value);
 /* ---- measurement helpers ----------------------------------------------------- */
 
 /* When enabled, the next transposes record per-pass GPU time (HIP events on
- * the launching stream); eithot_last_pass_times copies up to max of them (ms). */
+ * the launching stream); eithot_last_pass_times copies up to max of them (ms):
+ * one when the call ran as one whole pass ("whole" above). */
 void eithot_set_pass_timing(int enable);
 int eithot_last_pass_times(float* ms, int max);
 
