@@ -2,7 +2,9 @@
 // element sizes may all differ) transposed with one persistent launch per
 // decomposition-stage index, captured once in a HIP graph and replayed.
 //
-// Launch k runs pass k of every tensor whose plan has one; passes that
+// Tensors of several passes that fit a whole-permutation pass (whole.hpp) run
+// in one resident launch of all of them.  For the others, launch k runs pass
+// k of every tensor whose plan has one; passes that
 // cannot join a persistent launch (scratch-staged or 64-bit indexed) run as
 // their own launches right after launch k.  Every tensor's passes therefore
 // keep their order, and tensors never share footprints.
@@ -53,7 +55,9 @@ void free_stages(std::vector<LaunchStage>& v) {
 
 struct eithot_batch {
   std::vector<TensorReq> tensors;
-  std::vector<Plan> fwd, inv;
+  std::vector<Plan> fwd, inv;  // a tensor that the resident launch takes keeps no passes
+  std::vector<WholePass> fwd_whole, inv_whole;
+  WholeBatch* whole = nullptr;  // the resident launch, before the stages
   std::vector<LaunchStage> stages;
   char* scratch = nullptr;
   int64_t scratch_bytes = 0;
@@ -67,6 +71,7 @@ struct eithot_batch {
 
   ~eithot_batch() {
     free_stages(stages);
+    whole_batch_free(whole);
     if (exec) (void)hipGraphExecDestroy(exec);
     if (graph) (void)hipGraphDestroy(graph);
     if (scratch) (void)hipFree(scratch);
@@ -91,7 +96,36 @@ struct eithot_batch {
     return EITHOT_OK;
   }
 
-  int enqueue(const std::vector<LaunchStage>& st, const LaunchCfg& c, hipStream_t s) {
+  // The whole-permutation pass of a tensor whose plan has several passes
+  // (batched passes of small tensors wait for each other's launches, so one
+  // pass gains most here).
+  void choose_whole(const TensorReq& r, const std::vector<int64_t>& dims, const std::vector<int>& perm,
+                    const DeviceProfile& prof, Plan& plan, WholePass& w) {
+    w = WholePass();
+    if (!prof.whole || plan.ops.size() < 2) return;
+    w = plan_whole_batched(dims.data(), perm.data(), (int)dims.size(), r.elem, prof.cus, prof.lds_max);
+    if (w.mode == WHOLE_NONE) return;
+    plan.ops.clear();
+    plan.scratch_bytes = 0;
+  }
+
+  int build_whole(const std::vector<WholePass>& v, WholeBatch** out) {
+    std::vector<std::pair<const WholePass*, char*>> p;
+    for (size_t t = 0; t < v.size(); ++t)
+      if (v[t].mode != WHOLE_NONE) p.push_back({&v[t], tensors[t].dev});
+    // the largest regions first: the launch ends on short ones
+    std::stable_sort(p.begin(), p.end(), [](const auto& x, const auto& y) {
+      return x.first->g.tiles > y.first->g.tiles;
+    });
+    if (whole_batch_build(p, dev->whole_ctl, out) != hipSuccess)
+      return fail(EITHOT_ERR_NOMEM, "building the batch's resident pass failed");
+    return EITHOT_OK;
+  }
+
+  int enqueue(const WholeBatch* w, const std::vector<LaunchStage>& st, const LaunchCfg& c,
+              hipStream_t s) {
+    if (whole_batch_enqueue(w, s) != hipSuccess)
+      return fail(EITHOT_ERR_DEVICE, "batched resident launch failed");
     for (const LaunchStage& x : st) {
       if (batch_launch_enqueue(x.persistent, s) != hipSuccess)
         return fail(EITHOT_ERR_DEVICE, "batched launch failed");
@@ -141,14 +175,21 @@ int eithot_batch_build(eithot_batch* b, double alpha, int tune) {
   DeviceProfile prof = b->dev->profile();
   prof.cycle_shift = 0;  // batched cycle items move narrow cells word by word
   b->cfg = b->dev->launch_cfg();
+  {
+    std::lock_guard<std::mutex> lk(b->dev->enqueue_mu);
+    if (prof.whole && !b->dev->whole_init_locked()) prof.whole = 0;
+  }
   b->fwd.resize(n);
   b->inv.resize(n);
+  b->fwd_whole.resize(n);
+  b->inv_whole.resize(n);
   for (size_t t = 0; t < n; ++t) {
     const TensorReq& r = b->tensors[t];
     const int order = (int)r.dims.size();
     int rc = make_plan(r.dims.data(), r.perm.data(), order, r.elem, 1, alpha, prof, prof.reorder,
                        b->fwd[t]);
     if (rc) return fail(rc, "planning tensor %zu failed (%d)", t, rc);
+    b->choose_whole(r, r.dims, r.perm, prof, b->fwd[t], b->fwd_whole[t]);
     b->scratch_bytes = std::max(b->scratch_bytes, b->fwd[t].scratch_bytes);
     if (tune) {
       std::vector<int64_t> od(order);
@@ -160,6 +201,7 @@ int eithot_batch_build(eithot_batch* b, double alpha, int tune) {
       rc = make_plan(od.data(), ip.data(), order, r.elem, 1, alpha, prof, prof.reorder,
                      b->inv[t]);
       if (rc) return fail(rc, "planning inverse of tensor %zu failed (%d)", t, rc);
+      b->choose_whole(r, od, ip, prof, b->inv[t], b->inv_whole[t]);
       b->scratch_bytes = std::max(b->scratch_bytes, b->inv[t].scratch_bytes);
     }
   }
@@ -180,6 +222,8 @@ int eithot_batch_build(eithot_batch* b, double alpha, int tune) {
     (void)hipGetLastError();
     return fail(EITHOT_ERR_NOMEM, "batch scratch allocation failed");
   }
+  int rc = b->build_whole(b->fwd_whole, &b->whole);
+  if (rc) return rc;
   std::vector<Candidate> cands = {{b->cfg.lds_target, b->cfg.threads, 0}};
   if (tune) {
     cands.clear();
@@ -190,6 +234,8 @@ int eithot_batch_build(eithot_batch* b, double alpha, int tune) {
   float best_ms = 1e30f;
   Candidate best = cands[0];
   if (cands.size() > 1) {
+    WholeBatch* whole_inv = nullptr;
+    if ((rc = b->build_whole(b->inv_whole, &whole_inv))) return rc;
     hipEvent_t e0, e1, e2;
     (void)hipEventCreate(&e0);
     (void)hipEventCreate(&e1);
@@ -200,14 +246,19 @@ int eithot_batch_build(eithot_batch* b, double alpha, int tune) {
       cfg.threads = c.threads;
       cfg.threads_big = std::max(c.threads, 512);
       std::vector<LaunchStage> f, v;
-      int rc = b->build_stages(b->fwd, cfg, c.grid_per_cu, f);
+      rc = b->build_stages(b->fwd, cfg, c.grid_per_cu, f);
       if (!rc) rc = b->build_stages(b->inv, cfg, c.grid_per_cu, v);
       if (!rc) {
-        (void)hipEventRecord(e0, b->stream);
-        rc = b->enqueue(f, cfg, b->stream);
-        (void)hipEventRecord(e1, b->stream);
-        if (!rc) rc = b->enqueue(v, cfg, b->stream);
-        (void)hipEventRecord(e2, b->stream);
+        {
+          std::lock_guard<std::mutex> lk(b->dev->enqueue_mu);
+          if (b->whole || whole_inv) rc = b->dev->whole_begin_locked(b->stream);
+          (void)hipEventRecord(e0, b->stream);
+          if (!rc) rc = b->enqueue(b->whole, f, cfg, b->stream);
+          (void)hipEventRecord(e1, b->stream);
+          if (!rc) rc = b->enqueue(whole_inv, v, cfg, b->stream);
+          (void)hipEventRecord(e2, b->stream);
+          if (!rc && (b->whole || whole_inv)) rc = b->dev->whole_end_locked(b->stream);
+        }
         if (hipStreamSynchronize(b->stream) != hipSuccess) rc = EITHOT_ERR_DEVICE;
       }
       float ms = 0;
@@ -217,13 +268,16 @@ int eithot_batch_build(eithot_batch* b, double alpha, int tune) {
       }
       free_stages(f);
       free_stages(v);
+      if (!rc) rc = b->dev->whole_status();
       if (rc) {
         (void)hipEventDestroy(e0);
         (void)hipEventDestroy(e1);
         (void)hipEventDestroy(e2);
+        whole_batch_free(whole_inv);
         return rc;
       }
     }
+    whole_batch_free(whole_inv);
     (void)hipEventDestroy(e0);
     (void)hipEventDestroy(e1);
     (void)hipEventDestroy(e2);
@@ -233,7 +287,8 @@ int eithot_batch_build(eithot_batch* b, double alpha, int tune) {
   b->cfg.threads_big = std::max(best.threads, 512);
   b->grid_per_cu = best.grid_per_cu;
   b->inv.clear();
-  int rc = b->build_stages(b->fwd, b->cfg, b->grid_per_cu, b->stages);
+  b->inv_whole.clear();
+  rc = b->build_stages(b->fwd, b->cfg, b->grid_per_cu, b->stages);
   if (rc) return rc;
   for (const LaunchStage& st : b->stages)
     for (const auto& so : st.side)
@@ -242,7 +297,7 @@ int eithot_batch_build(eithot_batch* b, double alpha, int tune) {
   // capture the forward launches once; replays reuse the instantiated graph
   if (hipStreamBeginCapture(b->stream, hipStreamCaptureModeThreadLocal) != hipSuccess)
     return fail(EITHOT_ERR_DEVICE, "graph capture failed to start");
-  rc = b->enqueue(b->stages, b->cfg, b->stream);
+  rc = b->enqueue(b->whole, b->stages, b->cfg, b->stream);
   hipError_t e = hipStreamEndCapture(b->stream, &b->graph);
   if (rc) return rc;
   if (e != hipSuccess) return fail(EITHOT_ERR_DEVICE, "graph capture failed");
@@ -255,16 +310,28 @@ int eithot_batch_build(eithot_batch* b, double alpha, int tune) {
 int eithot_batch_run(eithot_batch* b, void* stream, int sync) {
   if (!b || !b->built) return fail(EITHOT_ERR_INVALID, "batch not built");
   hipStream_t s = stream ? (hipStream_t)stream : b->stream;
-  if (hipGraphLaunch(b->exec, s) != hipSuccess) return fail(EITHOT_ERR_DEVICE, "graph launch failed");
+  int rc = EITHOT_OK;
+  if (b->whole) {
+    if ((rc = b->dev->whole_status())) return rc;
+    std::lock_guard<std::mutex> lk(b->dev->enqueue_mu);
+    if (b->dev->whole_off)
+      return fail(EITHOT_ERR_DEVICE, "resident passes are off on this device: build the batch again");
+    if ((rc = b->dev->whole_begin_locked(s))) return rc;
+    if (hipGraphLaunch(b->exec, s) != hipSuccess)
+      return fail(EITHOT_ERR_DEVICE, "graph launch failed");
+    if ((rc = b->dev->whole_end_locked(s))) return rc;
+  } else if (hipGraphLaunch(b->exec, s) != hipSuccess) {
+    return fail(EITHOT_ERR_DEVICE, "graph launch failed");
+  }
   if (sync && hipStreamSynchronize(s) != hipSuccess)
     return fail(EITHOT_ERR_DEVICE, "batch execution failed");
-  return EITHOT_OK;
+  return sync && b->whole ? b->dev->whole_status() : EITHOT_OK;
 }
 
 int eithot_batch_info(const eithot_batch* b, int* launches, int64_t* scratch_bytes,
                       int* graph_captured) {
   if (!b) return fail(EITHOT_ERR_INVALID, "null batch");
-  int n = 0;
+  int n = b->whole ? 1 : 0;
   for (const auto& s : b->stages) n += batch_launch_count(s.persistent) + (int)s.side.size();
   if (launches) *launches = n;
   if (scratch_bytes) *scratch_bytes = b->scratch_bytes;

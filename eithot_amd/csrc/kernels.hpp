@@ -87,15 +87,20 @@ int64_t batch_launch_items(const BatchLaunch* L);
 int batch_launch_count(const BatchLaunch* L);  // kernel launches per enqueue
 
 // The whole-permutation pass `p` over the tensor at `data` (whole.hip).  A
-// resident pass whose workgroups do not meet within `patience` ticks of the
-// 100 MHz clock sets *host_failed and leaves the tensor indeterminate.
+// resident pass whose workgroups do not meet within ctl.patience sets
+// *ctl.host_failed and leaves the tensor indeterminate.
 struct WholePass;
-struct WholeTurn {
-  uint32_t pass = 0;  // number of this resident pass on its device, from 1, never 0
-  uint64_t patience = 0;
-  uint32_t* host_failed = nullptr;
-};
-hipError_t launch_whole(const WholePass& p, char* data, const WholeTurn& turn, hipStream_t stream);
+struct WholeCtl;
+hipError_t launch_whole(const WholePass& p, char* data, const WholeCtl& ctl, hipStream_t stream);
+// the current device's words for single tensors (fills ctl's pointers to them)
+hipError_t whole_ctl_device(WholeCtl& ctl);
+// Resident passes (plan_whole_batched) of many tensors in one launch, with
+// words of their own; ctl gives the failure words and the patience.
+struct WholeBatch;
+hipError_t whole_batch_build(const std::vector<std::pair<const WholePass*, char*>>& passes,
+                             const WholeCtl& ctl, WholeBatch** out);
+hipError_t whole_batch_enqueue(const WholeBatch* w, hipStream_t stream);
+void whole_batch_free(WholeBatch* w);
 hipError_t configure_whole(int64_t bytes);
 
 // Raise the dynamic-LDS limit of every pass kernel to `bytes` (once per device).

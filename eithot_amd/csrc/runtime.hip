@@ -250,21 +250,44 @@ bool stream_captured(hipStream_t stream) {
 bool Device::takes_whole_locked(const Plan& plan, hipStream_t stream) {
   if (!plan.whole) return false;
   if (plan.whole->mode == WHOLE_ORBIT) return true;
-  if (whole_off || stream_captured(stream)) return false;
-  if (!whole_failed) {
-    if (hipHostMalloc((void**)&whole_failed, sizeof(uint32_t), hipHostMallocDefault) != hipSuccess) {
-      (void)hipGetLastError();
-      whole_failed = nullptr;
-      return false;
-    }
-    *whole_failed = 0;
-  }
-  if (!whole_ready && hipEventCreateWithFlags(&whole_ready, hipEventDisableTiming) != hipSuccess) {
+  return !whole_off && !stream_captured(stream) && whole_init_locked();
+}
+
+bool Device::whole_init_locked() {
+  if (whole_ready) return !whole_off;
+  WholeCtl c;
+  c.patience = kWholePatience;
+  hipEvent_t ev = nullptr;
+  if (whole_off || whole_ctl_device(c) != hipSuccess ||
+      hipHostMalloc((void**)&c.host_failed, sizeof(uint32_t), hipHostMallocDefault) != hipSuccess ||
+      hipEventCreateWithFlags(&ev, hipEventDisableTiming) != hipSuccess) {
     (void)hipGetLastError();
-    whole_ready = nullptr;
+    whole_off = true;
     return false;
   }
+  *c.host_failed = 0;
+  whole_ctl = c;
+  whole_ready = ev;
   return true;
+}
+
+// Passes on the null stream follow each other by themselves; the event is
+// recorded behind them only when a call on another stream needs it (the null
+// stream outlives every call, other streams may not).
+int Device::whole_begin_locked(hipStream_t stream) {
+  if (!stream && !whole_elsewhere) return EITHOT_OK;
+  if (!whole_elsewhere && hipEventRecord(whole_ready, nullptr) != hipSuccess)
+    return fail(EITHOT_ERR_DEVICE, "hipEventRecord failed");
+  if (hipStreamWaitEvent(stream, whole_ready, 0) != hipSuccess)
+    return fail(EITHOT_ERR_DEVICE, "hipStreamWaitEvent failed");
+  return EITHOT_OK;
+}
+
+int Device::whole_end_locked(hipStream_t stream) {
+  whole_elsewhere = stream != nullptr;
+  if (stream && hipEventRecord(whole_ready, stream) != hipSuccess)
+    return fail(EITHOT_ERR_DEVICE, "hipEventRecord failed");
+  return EITHOT_OK;
 }
 
 int Device::launch_whole_locked(const Plan& plan, char* data, hipStream_t stream) {
@@ -274,33 +297,18 @@ int Device::launch_whole_locked(const Plan& plan, char* data, hipStream_t stream
   if (chain && plan.table_bytes > 0 && plan.device_table_bytes(id) < plan.table_bytes)
     for (const Op& o : plan.ops)
       if (prepare_op(o) != hipSuccess) return fail(EITHOT_ERR_DEVICE, "uploading a pass table failed");
-  // Passes on the null stream follow each other by themselves; the event is
-  // recorded behind them only when a call on another stream needs it (the
-  // null stream outlives every call, other streams may not).
-  if (chain && (stream || whole_elsewhere)) {
-    if (!whole_elsewhere && hipEventRecord(whole_ready, nullptr) != hipSuccess)
-      return fail(EITHOT_ERR_DEVICE, "hipEventRecord failed");
-    if (hipStreamWaitEvent(stream, whole_ready, 0) != hipSuccess)
-      return fail(EITHOT_ERR_DEVICE, "hipStreamWaitEvent failed");
-  }
-  WholeTurn& t = whole_turn;
-  if (chain) {
-    if (++t.pass == 0) ++t.pass;
-    t.patience = kWholePatience;
-    t.host_failed = whole_failed;
-  }
-  const hipError_t e = launch_whole(*plan.whole, data, t, stream);
+  int rc = chain ? whole_begin_locked(stream) : EITHOT_OK;
+  if (rc) return rc;
+  const hipError_t e = launch_whole(*plan.whole, data, whole_ctl, stream);
   if (e != hipSuccess)
     return fail(EITHOT_ERR_DEVICE, "whole pass launch failed: %s", hipGetErrorString(e));
-  if (chain) whole_elsewhere = stream != nullptr;
-  if (chain && stream && hipEventRecord(whole_ready, stream) != hipSuccess)
-    return fail(EITHOT_ERR_DEVICE, "hipEventRecord failed");
-  return EITHOT_OK;
+  return chain ? whole_end_locked(stream) : EITHOT_OK;
 }
 
 int Device::whole_status() {
   std::lock_guard<std::mutex> lk(enqueue_mu);
-  if (whole_off || !whole_failed || !*(volatile uint32_t*)whole_failed) return EITHOT_OK;
+  if (whole_off || !whole_ctl.host_failed || !*(volatile uint32_t*)whole_ctl.host_failed)
+    return EITHOT_OK;
   whole_off = true;
   return fail(EITHOT_ERR_DEVICE,
               "a resident pass gave up waiting for its workgroups; the tensors of calls since the "

@@ -37,13 +37,12 @@ struct Device {
   hipEvent_t arena_ready = nullptr;  // recorded after the last pass that used the arena
   // Resident whole-permutation passes share the chip with no other of their
   // kind (whole.hip): each waits, on the device, for the one before.  Once
-  // one has given up waiting (*whole_failed, written by the kernel) the
+  // one has given up waiting (*whole_ctl.host_failed, written by the kernel) the
   // device runs ordinary passes only.  All under enqueue_mu.
   hipEvent_t whole_ready = nullptr;
   bool whole_elsewhere = false;      // the last one ran on a stream other than the null stream
-  uint32_t* whole_failed = nullptr;  // pinned host memory
   bool whole_off = false;
-  WholeTurn whole_turn;
+  WholeCtl whole_ctl;
   // device bytes of the pass tables uploaded for plans of this cache (and
   // not yet freed; an evicted plan a request still holds counts until freed)
   std::atomic<int64_t> cached_tables{0};
@@ -73,6 +72,11 @@ struct Device {
   // whole-permutation pass, and the launch of it.  Resident passes are left
   // out of stream captures (a replay could not be chained).
   bool takes_whole_locked(const Plan& plan, hipStream_t stream);
+  // Resident passes on `stream` go between these two; whole_init_locked
+  // comes before the first (false: the device runs none).
+  bool whole_init_locked();
+  int whole_begin_locked(hipStream_t stream);
+  int whole_end_locked(hipStream_t stream);
   int launch_whole_locked(const Plan& plan, char* data, hipStream_t stream);
   // Reports (once) that a resident pass gave up: its tensor's contents are
   // indeterminate.  EITHOT_OK otherwise.

@@ -1,6 +1,8 @@
 // gfx950 kernels of the whole-permutation passes (whole.hpp).
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
+
 #include "kernels.hpp"
 #include "whole.hpp"
 
@@ -206,20 +208,10 @@ __device__ __forceinline__ void tile_store(const WholeGeom& g, const WholeTile& 
 // ---------------------------------------------------------------------------
 // resident form
 // ---------------------------------------------------------------------------
-// Words in which a device's resident passes count the workgroups that have
-// loaded their tiles: 16 counters per region (each on a line of its own: one
-// address takes about 30 ns per addition) and a root that the last workgroup
-// of each adds to, all zero between passes, and the number of the last pass
-// in which the region was complete.
-constexpr uint32_t kSubs = 16;
-struct WholeCtl {
-  uint32_t failed, pad[31];
-  uint32_t open[kWholeRegions];
-  uint32_t root[kWholeRegions];
-  uint32_t sub[kSubs][kWholeRegions];
-};
-__device__ WholeCtl g_ctl;
-
+// Counts workgroup t of the n of a region; true for the last one.  A region
+// has 16 counters (each on a line of its own: one address takes about 30 ns
+// per addition) and a root that the last workgroup of each adds to, all zero
+// between passes.
 __device__ __forceinline__ uint32_t ctl_add(uint32_t* p, uint32_t v) {
   return __hip_atomic_fetch_add(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
@@ -229,38 +221,36 @@ __device__ __forceinline__ uint32_t ctl_get(uint32_t* p) {
 __device__ __forceinline__ void ctl_set(uint32_t* p, uint32_t v) {
   __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
-
-// Counts workgroup t of the n of region b; true for the last one.
-__device__ __forceinline__ bool ctl_arrive(uint32_t b, uint32_t t, uint32_t n) {
-  const uint32_t subs = n <= kSubs ? 1 : kSubs;
+__device__ __forceinline__ bool ctl_arrive(const WholeCtl& c, uint32_t slot, uint32_t t, uint32_t n) {
+  const uint32_t subs = n <= kWholeSubs ? 1 : kWholeSubs;
   const uint32_t j = t % subs, members = (n - j + subs - 1) / subs;
-  if (ctl_add(&g_ctl.sub[j][b], 1) != members - 1) return false;
-  ctl_set(&g_ctl.sub[j][b], 0);
+  uint32_t* sub = c.sub + (uint64_t)j * c.slots + slot;
+  if (ctl_add(sub, 1) != members - 1) return false;
+  ctl_set(sub, 0);
   if (subs == 1) return true;
-  if (ctl_add(&g_ctl.root[b], 1) != subs - 1) return false;
-  ctl_set(&g_ctl.root[b], 0);
+  if (ctl_add(c.root + slot, 1) != subs - 1) return false;
+  ctl_set(c.root + slot, 0);
   return true;
 }
 
-// One tile per workgroup.  The tiles of a region have consecutive block
-// indices, and workgroups start in that order on each XCD, so those of the
-// earliest unfinished region all run as soon as as many as it has tiles are
-// resident, which the planner keeps to half of the chip's room; they wait
-// for nobody else.  Launches of this kernel on one device follow each other
-// (the runtime chains them), so no two share that room.  No data passes
-// between workgroups: the counters only order a region's loads, which are
-// complete once in LDS, before its stores, so they need no cache flush.  The
-// wait is bounded all the same: after `patience` ticks of the 100 MHz clock
-// a workgroup reports a failure and leaves without storing, and so do those
-// after it.
-template <int WL, bool MULTI, int ND>
-__global__ __launch_bounds__(1024) void k_resident(WholeGeom g, char* data, uint32_t pass,
-                                                   uint64_t patience, uint32_t* host_failed) {
-  extern __shared__ __align__(16) unsigned char lds[];
+// Tiles t * per .. of region b, meeting its region's other workgroups at
+// `slot`.  The first is held in LDS, a second one in registers until the
+// first is stored.  No data passes between workgroups: the counters only
+// order a region's loads, which are complete once in LDS or waited for,
+// before its stores, so they need no cache flush.  The wait is bounded: after
+// `patience` ticks of the 100 MHz clock a workgroup reports a failure and
+// leaves without storing, and so do those after it.
+template <int WL, bool MULTI, int ND, bool PAIR>
+__device__ __forceinline__ void resident_body(const WholeGeom& g, char* data, uint32_t b, uint32_t t,
+                                              uint32_t slot, const WholeCtl& c,
+                                              unsigned char* lds) {
   uint32_t* ctl = reinterpret_cast<uint32_t*>(lds);
-  const uint32_t b = g.ftiles.div(blockIdx.x), t = blockIdx.x - b * g.tiles;
-  const WholeTile x = whole_tile<ND>(g, whole_nth(g, t));
-  const uint64_t region = (uint64_t)b * g.region;
+  // the region is complete when this word changes
+  uint32_t closed = 0;
+  if (threadIdx.x == 0) closed = ctl_get(c.open + slot);
+  const WholeTile x = whole_tile<ND>(g, whole_nth(g, PAIR ? t * g.per : t));
+  const uint64_t region = (uint64_t)b * g.region, room = g.B * g.region - region;
+  char* base = data + region;
   const Areas a = areas(g, lds);
   list_in<ND>(g, x, a);
   list_out<ND>(g, x, a);
@@ -270,22 +260,35 @@ __global__ __launch_bounds__(1024) void k_resident(WholeGeom g, char* data, uint
   for (Walk k(g.fcin); k.rho < g.nin;) {
     V16 v[8];
     uint32_t at[8];
-    get_chunks(g, data + region + x.in, g.B * g.region - region - x.in, run_bytes, a, k, v, at);
+    get_chunks(g, base + x.in, room - x.in, run_bytes, a, k, v, at);
     put_chunks<WL>(a, v, at);
+  }
+  const bool second = PAIR && g.per == 2 && 2 * t + 1 < g.tiles;
+  WholeTile y = x;
+  V16 hv[8];
+  uint32_t hat[8];
+  if (second) {
+    y = whole_tile<ND>(g, whole_nth(g, 2 * t + 1));
+    __syncthreads();  // the list of x's input runs has been read
+    list_in<ND>(g, y, a);
+    __syncthreads();
+    Walk k(g.fcin);
+    get_chunks(g, base + y.in, room - y.in, whole_len_in<ND>(g, y) << WL, a, k, hv, hat);
+    __builtin_amdgcn_s_waitcnt(0);
   }
   __syncthreads();
   if (threadIdx.x == 0) {
     uint32_t ok = 1;
-    if (ctl_arrive(b, t, g.tiles)) {
-      ctl_set(&g_ctl.open[b], pass);
+    if (ctl_arrive(c, slot, t, g.wgs)) {
+      ctl_set(c.open + slot, closed + 1);
     } else {
       const uint64_t t0 = __builtin_amdgcn_s_memrealtime();
       for (;;) {
-        const uint32_t failed = ctl_get(&g_ctl.failed), now = ctl_get(&g_ctl.open[b]);
-        if (!failed && now == pass) break;
-        if (failed || __builtin_amdgcn_s_memrealtime() - t0 > patience) {
-          ctl_set(&g_ctl.failed, 1);
-          __hip_atomic_store(host_failed, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        const uint32_t failed = ctl_get(c.failed), now = ctl_get(c.open + slot);
+        if (!failed && now != closed) break;
+        if (failed || __builtin_amdgcn_s_memrealtime() - t0 > c.patience) {
+          ctl_set(c.failed, 1);
+          __hip_atomic_store(c.host_failed, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
           ok = 0;
           break;
         }
@@ -295,8 +298,64 @@ __global__ __launch_bounds__(1024) void k_resident(WholeGeom g, char* data, uint
     ctl[0] = ok;
   }
   __syncthreads();
-  if (ctl[0]) tile_store<WL, MULTI, ND>(g, x, data + region + x.out, a);
+  if (!ctl[0]) return;
+  tile_store<WL, MULTI, ND>(g, x, base + x.out, a);
+  if (second) {
+    __syncthreads();  // x has been read out of LDS, and its lists
+    put_chunks<WL>(a, hv, hat);
+    list_out<ND>(g, y, a);
+    __syncthreads();
+    tile_store<WL, MULTI, ND>(g, y, base + y.out, a);
+  }
 }
+
+// One tile, or two, per workgroup.  The workgroups of a region have
+// consecutive block indices, and workgroups start in that order on each XCD, so those of the
+// earliest unfinished region all run as soon as that many are resident, which the planner keeps to half of the chip's room; they wait
+// for nobody else.  Launches of resident passes on one device follow each
+// other (the runtime chains them), so no two share that room.
+template <int WL, bool MULTI, int ND, bool PAIR>
+__global__ __launch_bounds__(1024) void k_resident(WholeGeom g, char* data, WholeCtl c) {
+  extern __shared__ __align__(16) unsigned char lds[];
+  const uint32_t b = g.fwgs.div(blockIdx.x);
+  resident_body<WL, MULTI, ND, PAIR>(g, data, b, blockIdx.x - b * g.wgs, b, c, lds);
+}
+
+// The same over the regions of many tensors: workgroup i takes item i.
+struct WholeItem {
+  uint32_t op, b, t, slot;
+};
+struct WholeOp {
+  WholeGeom g;
+  char* data;
+  int variant;  // log2(word) * 4 + (runs over several dims) * 2 + (at most 4 dims)
+};
+__global__ __launch_bounds__(256) void k_resident_batch(const WholeOp* __restrict__ ops,
+                                                        const WholeItem* __restrict__ items,
+                                                        WholeCtl c) {
+  extern __shared__ __align__(16) unsigned char lds[];
+  const WholeItem i = items[blockIdx.x];
+  const WholeOp& o = ops[i.op];
+  const WholeGeom& g = o.g;
+#define EH_WHOLE(WL, MULTI, ND)                                                       \
+  case (WL)*4 + (MULTI)*2 + (ND == 4):                                                \
+    resident_body<WL, MULTI, ND, true>(g, o.data, i.b, i.t, i.slot, c, lds);          \
+    break;
+#define EH_WHOLE_W(WL)                                                                \
+  EH_WHOLE(WL, false, 4) EH_WHOLE(WL, true, 4) EH_WHOLE(WL, false, 8) EH_WHOLE(WL, true, 8)
+  switch (o.variant) {
+    EH_WHOLE_W(0)
+    EH_WHOLE_W(1)
+    EH_WHOLE_W(2)
+    EH_WHOLE_W(3)
+    EH_WHOLE_W(4)
+  }
+#undef EH_WHOLE_W
+#undef EH_WHOLE
+}
+
+// the words of a device's resident passes over single tensors
+__device__ uint32_t g_ctl[whole_ctl_words(kWholeRegions)];
 
 // ---------------------------------------------------------------------------
 // orbit form
@@ -352,31 +411,35 @@ __global__ __launch_bounds__(512) void k_orbit(WholeGeom g, char* data) {
 }
 
 template <int WL, bool MULTI, int ND>
-hipError_t launch_i(const WholePass& p, char* data, const WholeTurn& turn,
-                    hipStream_t st) {
-  const dim3 grid((uint32_t)(p.g.tiles * p.g.B)), block(p.threads);
+hipError_t launch_i(const WholePass& p, char* data, const WholeCtl& c, hipStream_t st) {
+  const dim3 block(p.threads);
+  const uint32_t per_region = p.mode == WHOLE_ORBIT ? p.g.tiles : p.g.wgs;
+  const dim3 grid((uint32_t)(per_region * p.g.B));
   if (p.mode == WHOLE_ORBIT)
     hipLaunchKernelGGL((k_orbit<WL, MULTI, ND>), grid, block, (size_t)p.lds, st, p.g, data);
+  else if (p.g.per == 2)
+    hipLaunchKernelGGL((k_resident<WL, MULTI, ND, true>), grid, block, (size_t)p.lds, st, p.g, data, c);
   else
-    hipLaunchKernelGGL((k_resident<WL, MULTI, ND>), grid, block, (size_t)p.lds, st, p.g, data, turn.pass,
-                       turn.patience, turn.host_failed);
+    hipLaunchKernelGGL((k_resident<WL, MULTI, ND, false>), grid, block, (size_t)p.lds, st, p.g, data, c);
   return hipGetLastError();
 }
 template <int WL>
-hipError_t launch_w(const WholePass& p, char* data, const WholeTurn& turn,
-                    hipStream_t st) {
+hipError_t launch_w(const WholePass& p, char* data, const WholeCtl& c, hipStream_t st) {
   const bool multi = p.g.jout > 1;
   if (p.g.r <= 4)
-    return multi ? launch_i<WL, true, 4>(p, data, turn, st)
-                 : launch_i<WL, false, 4>(p, data, turn, st);
-  return multi ? launch_i<WL, true, kWholeDims>(p, data, turn, st)
-               : launch_i<WL, false, kWholeDims>(p, data, turn, st);
+    return multi ? launch_i<WL, true, 4>(p, data, c, st) : launch_i<WL, false, 4>(p, data, c, st);
+  return multi ? launch_i<WL, true, kWholeDims>(p, data, c, st)
+               : launch_i<WL, false, kWholeDims>(p, data, c, st);
 }
 template <int WL>
 void configure_w(int64_t bytes, hipError_t& e) {
-  for (const void* fn : {(const void*)k_resident<WL, false, 4>, (const void*)k_resident<WL, true, 4>,
-                         (const void*)k_resident<WL, false, kWholeDims>,
-                         (const void*)k_resident<WL, true, kWholeDims>}) {
+  for (const void* fn :
+       {(const void*)k_resident<WL, false, 4, false>, (const void*)k_resident<WL, true, 4, false>,
+        (const void*)k_resident<WL, false, kWholeDims, false>,
+        (const void*)k_resident<WL, true, kWholeDims, false>,
+        (const void*)k_resident<WL, false, 4, true>, (const void*)k_resident<WL, true, 4, true>,
+        (const void*)k_resident<WL, false, kWholeDims, true>,
+        (const void*)k_resident<WL, true, kWholeDims, true>}) {
     const hipError_t r = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
     if (r != hipSuccess) e = r;
   }
@@ -384,15 +447,21 @@ void configure_w(int64_t bytes, hipError_t& e) {
 
 }  // namespace
 
-hipError_t launch_whole(const WholePass& p, char* data, const WholeTurn& turn,
-                        hipStream_t st) {
+hipError_t launch_whole(const WholePass& p, char* data, const WholeCtl& ctl, hipStream_t st) {
   switch (p.g.w) {
-    case 16: return launch_w<4>(p, data, turn, st);
-    case 8: return launch_w<3>(p, data, turn, st);
-    case 4: return launch_w<2>(p, data, turn, st);
-    case 2: return launch_w<1>(p, data, turn, st);
-    default: return launch_w<0>(p, data, turn, st);
+    case 16: return launch_w<4>(p, data, ctl, st);
+    case 8: return launch_w<3>(p, data, ctl, st);
+    case 4: return launch_w<2>(p, data, ctl, st);
+    case 2: return launch_w<1>(p, data, ctl, st);
+    default: return launch_w<0>(p, data, ctl, st);
   }
+}
+
+hipError_t whole_ctl_device(WholeCtl& c) {
+  void* p = nullptr;
+  const hipError_t e = hipGetSymbolAddress(&p, HIP_SYMBOL(g_ctl));
+  if (e == hipSuccess) whole_ctl_at(c, (uint32_t*)p, kWholeRegions);
+  return e;
 }
 
 hipError_t configure_whole(int64_t bytes) {
@@ -403,6 +472,75 @@ hipError_t configure_whole(int64_t bytes) {
   configure_w<3>(bytes, e);
   configure_w<4>(bytes, e);
   return e;
+}
+
+// ---------------------------------------------------------------------------
+// many tensors in one launch
+// ---------------------------------------------------------------------------
+struct WholeBatch {
+  char* mem = nullptr;  // ops, items and counters
+  WholeOp* ops = nullptr;
+  WholeItem* items = nullptr;
+  WholeCtl ctl;
+  uint32_t grid = 0;
+  int64_t lds = 0;
+};
+
+hipError_t whole_batch_build(const std::vector<std::pair<const WholePass*, char*>>& passes,
+                             const WholeCtl& ctl, WholeBatch** out) {
+  *out = nullptr;
+  std::vector<WholeOp> ops;
+  std::vector<WholeItem> items;
+  uint64_t slots = 0;
+  int64_t lds = 0;
+  for (const auto& p : passes) {
+    const WholeGeom& g = p.first->g;
+    const uint32_t op = (uint32_t)ops.size();
+    int wl = 0;
+    while ((1u << wl) < g.w) ++wl;
+    ops.push_back({g, p.second, wl * 4 + (g.jout > 1 ? 2 : 0) + (g.r <= 4 ? 1 : 0)});
+    lds = std::max(lds, p.first->lds);
+    for (uint32_t b = 0; b < g.B; ++b, ++slots)
+      for (uint32_t t = 0; t < g.wgs; ++t) items.push_back({op, b, t, (uint32_t)slots});
+  }
+  if (items.empty()) return hipSuccess;
+  if (items.size() >= (1ull << 31)) return hipErrorInvalidValue;
+  auto up = [](size_t n) { return (n + 255) / 256 * 256; };
+  const size_t ob = up(ops.size() * sizeof(WholeOp)), ib = up(items.size() * sizeof(WholeItem));
+  const size_t cb = whole_ctl_words((uint32_t)slots) * sizeof(uint32_t);
+  auto* w = new WholeBatch;
+  hipError_t e = hipMalloc((void**)&w->mem, ob + ib + cb);
+  if (e == hipSuccess)
+    e = hipMemcpy(w->mem, ops.data(), ops.size() * sizeof(WholeOp), hipMemcpyHostToDevice);
+  if (e == hipSuccess)
+    e = hipMemcpy(w->mem + ob, items.data(), items.size() * sizeof(WholeItem), hipMemcpyHostToDevice);
+  if (e == hipSuccess) e = hipMemset(w->mem + ob + ib, 0, cb);
+  if (e == hipSuccess) e = hipStreamSynchronize(nullptr);
+  if (e != hipSuccess) {
+    whole_batch_free(w);
+    return e;
+  }
+  w->ops = (WholeOp*)w->mem;
+  w->items = (WholeItem*)(w->mem + ob);
+  w->ctl = ctl;
+  whole_ctl_at(w->ctl, (uint32_t*)(w->mem + ob + ib), (uint32_t)slots);
+  w->grid = (uint32_t)items.size();
+  w->lds = lds;
+  *out = w;
+  return hipSuccess;
+}
+
+hipError_t whole_batch_enqueue(const WholeBatch* w, hipStream_t st) {
+  if (!w) return hipSuccess;
+  hipLaunchKernelGGL(k_resident_batch, dim3(w->grid), dim3(kWholeBatchThreads), (size_t)w->lds, st,
+                     w->ops, w->items, w->ctl);
+  return hipGetLastError();
+}
+
+void whole_batch_free(WholeBatch* w) {
+  if (!w) return;
+  if (w->mem) (void)hipFree(w->mem);
+  delete w;
 }
 
 }  // namespace eithot

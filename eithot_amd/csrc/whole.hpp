@@ -54,6 +54,8 @@ struct WholeGeom {
   FD32 ft[kWholeDims], oft[kWholeDims];    // tile extents, input and output order
   FD32 fcin, fcout;                        // 16-byte chunks per run
   FD32 ftiles;
+  uint32_t per = 1, wgs = 0;     // resident: tiles one workgroup holds (1 or 2), workgroups per region
+  FD32 fwgs;
   // Order in which workgroups take a matrix's tiles: along dim 0 within
   // groups of sg tiles (the last group: slast), then along dim 1, then the
   // next group.  sg = 0: index order.
@@ -209,11 +211,36 @@ EH_HD uint32_t whole_elem(const WholeGeom& g, uint32_t p) {
   return l;
 }
 
+// Where resident passes meet: per region kWholeSubs counters, a root counter
+// (zero between passes) and a word that the region's last workgroup steps.
+constexpr uint32_t kWholeSubs = 16;
+struct WholeCtl {
+  uint32_t* failed = nullptr;  // set by a workgroup that gave up waiting
+  uint32_t *open = nullptr, *root = nullptr, *sub = nullptr;
+  uint32_t slots = 0;                // regions the words serve
+  uint64_t patience = 0;             // ticks of the 100 MHz clock
+  uint32_t* host_failed = nullptr;   // pinned host word, set along with *failed
+};
+constexpr uint64_t whole_ctl_words(uint32_t slots) { return 32 + (uint64_t)slots * (2 + kWholeSubs); }
+inline void whole_ctl_at(WholeCtl& c, uint32_t* words, uint32_t slots) {
+  c.failed = words;
+  c.open = words + 32;
+  c.root = c.open + slots;
+  c.sub = c.root + slots;
+  c.slots = slots;
+}
+
 // Plans the whole-permutation pass of a tensor (perm1 1-based) for a chip of
 // `cus` CUs with lds_max bytes of LDS each; mode WHOLE_NONE when neither
 // form fits.  `passes` is the pass count of the tensor's ordinary plan, and
 // `weak` whether its only pass, when there is one, is worth replacing.
 WholePass plan_whole(const int64_t* dims, const int* perm1, int rank, size_t elem, int cus,
                      int64_t lds_max, int passes, bool weak);
+
+// The resident pass of a tensor among many in one launch: 32 KiB tiles,
+// workgroups of kWholeBatchThreads.
+constexpr int kWholeBatchThreads = 256;
+WholePass plan_whole_batched(const int64_t* dims, const int* perm1, int rank, size_t elem, int cus,
+                             int64_t lds_max);
 
 }  // namespace eithot

@@ -168,9 +168,10 @@ bool build(const Canon& c, const std::vector<int64_t>& t, WholeGeom& g) {
 // Tile extents within `cap` bytes of LDS: the shorter of the input and the
 // output run is doubled (its first dim that is not whole) while it fits; an
 // extent then shrinks to what its tile count needs, in whole 16-byte chunks
-// for the runs' last dims.  Dims of one class keep one extent.
+// for the runs' last dims.  Dims of one class keep one extent.  `tight` also
+// grows by half where doubling does not fit: fuller tiles, fewer whole lines.
 bool choose(const Canon& c, const std::vector<int>& cls, int64_t cap, int64_t max_chunks,
-            WholeGeom& g) {
+            WholeGeom& g, bool tight = false) {
   const int r = (int)c.d.size();
   std::vector<int64_t> t(r, 1);
   if (!build(c, t, g)) return false;
@@ -191,14 +192,18 @@ bool choose(const Canon& c, const std::vector<int>& cls, int64_t cap, int64_t ma
     for (int k = 0; k < r; ++k) {
       const int a = out ? c.p[k] : k;
       if (t[a] == c.d[a]) continue;
-      std::vector<int64_t> v = t;
-      set(v, a, std::min<int64_t>(c.d[a], 2 * t[a]));
-      WholeGeom h;
-      if (!build(c, v, h) || (int64_t)whole_lds_bytes(h) > cap ||
-          (int64_t)h.nin * h.fcin.d > max_chunks)
-        return false;
-      t = v;
-      return true;
+      for (int64_t f = 8; f > 4; f -= 2) {  // twice, then half as much again
+        std::vector<int64_t> v = t;
+        set(v, a, std::min<int64_t>(c.d[a], (f * t[a] + 3) / 4));
+        WholeGeom h;
+        if (v[a] > t[a] && build(c, v, h) && (int64_t)whole_lds_bytes(h) <= cap &&
+            (int64_t)h.nin * h.fcin.d <= max_chunks) {
+          t = v;
+          return true;
+        }
+        if (!tight) break;
+      }
+      return false;
     }
     return false;
   };
@@ -240,9 +245,36 @@ void order_tiles(WholeGeom& g) {
   g.fslast.init(g.slast);
 }
 
+void per_workgroup(WholeGeom& g, uint32_t per) {
+  g.per = per;
+  g.wgs = (g.tiles + per - 1) / per;
+  g.fwgs.init(g.wgs);
+}
+
 int64_t short_run(const WholeGeom& g) { return (int64_t)std::min(g.len_in, g.len_out) * g.w; }
 
 }  // namespace
+
+WholePass plan_whole_batched(const int64_t* dims, const int* perm1, int rank, size_t elem, int cus,
+                             int64_t lds_max) {
+  WholePass none, w;
+  Canon c;
+  if (!canonical(dims, perm1, rank, elem, c) || c.B > (int64_t)kWholeRegions) return none;
+  std::vector<int> cls(c.d.size());
+  for (size_t k = 0; k < cls.size(); ++k) cls[k] = (int)k;
+  constexpr int64_t kLds = 38 * 1024;  // of every workgroup of the launch
+  if (kLds > lds_max || !choose(c, cls, kLds, kWholeBatchThreads * kWholeHold, w.g, true)) return none;
+  // large regions: two tiles per workgroup, so that fewer of them wait for
+  // the rest of their region to start
+  per_workgroup(w.g, w.g.tiles > 16 ? 2 : 1);
+  const int64_t slots = (int64_t)cus * std::min<int64_t>(lds_max / kLds, 2048 / kWholeBatchThreads);
+  if ((int64_t)w.g.wgs > slots / 2 || short_run(w.g) < 32) return none;
+  w.threads = kWholeBatchThreads;
+  w.lds = (whole_lds_bytes(w.g) + 127) / 128 * 128;
+  w.mode = WHOLE_RESIDENT;
+  order_tiles(w.g);
+  return w;
+}
 
 WholePass plan_whole(const int64_t* dims, const int* perm1, int rank, size_t elem, int cus,
                      int64_t lds_max, int passes, bool weak) {
@@ -252,27 +284,35 @@ WholePass plan_whole(const int64_t* dims, const int* perm1, int rank, size_t ele
   const int r = (int)c.d.size();
   if (passes < 2 && !weak) return none;
 
+  struct Step {
+    int64_t lds;  // KiB
+    int threads;
+    uint32_t per;
+  };
+  constexpr Step kSteps[] = {{6, 256, 1},  {10, 256, 1},  {19, 256, 1},  {38, 256, 1},
+                             {78, 512, 1}, {156, 1024, 1}, {156, 1024, 2}};
   // resident: tiles as small as keeps the workgroups of a small tensor below
   // three per CU (77 KB: 17 -> 9.5 us, 4.4 MB: 33 -> 13 us, 1 MB of bytes:
   // 59 -> 10 us against the ordinary passes; meeting costs 2 to 5 us), and
   // 64 KiB tiles, two workgroups per CU, for larger ones and batches
   // (210 MB in regions of 3.6 MB: 158 -> 114 us; 32 KiB tiles 117, 128 KiB
-  // 132).  A region takes at most half of the workgroups the chip holds, so
+  // 132).  Where a region does not fit so, workgroups hold a second tile in
+  // registers.  A region takes at most half of the workgroups the chip holds, so
   // that two processes can always run theirs.
   if (c.B <= (int64_t)kWholeRegions) {
     std::vector<int> cls(r);
     for (int k = 0; k < r; ++k) cls[k] = k;
-    for (int64_t cap : {6, 10, 19, 38, 78, 156}) {
-      if (cap * 1024 > lds_max) break;
-      const int threads = cap <= 38 ? 256 : cap <= 78 ? 512 : 1024;
-      if (!choose(c, cls, cap * 1024, threads * kWholeHold, w.g)) continue;
+    for (const Step& st : kSteps) {
+      if (st.lds * 1024 > lds_max) break;
+      if (!choose(c, cls, st.lds * 1024, st.threads * kWholeHold, w.g)) continue;
       const int64_t lds = (whole_lds_bytes(w.g) + 127) / 128 * 128;
-      const int64_t slots = (int64_t)cus * std::min<int64_t>(lds_max / lds, 2048 / threads);
-      if ((int64_t)w.g.tiles > slots / 2) continue;
-      if (cap <= 38 && c.B * (int64_t)w.g.tiles > 3 * cus) continue;
+      const int64_t slots = (int64_t)cus * std::min<int64_t>(lds_max / lds, 2048 / st.threads);
+      per_workgroup(w.g, st.per);
+      if ((int64_t)w.g.wgs > slots / 2) continue;
+      if (st.lds <= 38 && c.B * (int64_t)w.g.tiles > 3 * cus) continue;
       const bool big = (uint64_t)c.B * w.g.region > (64ull << 20);
       if (short_run(w.g) < (big ? 128 : 32)) continue;
-      w.threads = threads;
+      w.threads = st.threads;
       w.lds = lds;
       w.mode = WHOLE_RESIDENT;
       order_tiles(w.g);
