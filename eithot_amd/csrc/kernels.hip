@@ -1978,34 +1978,14 @@ const void* cycle_table_device(const CycleTable& t, hipError_t* err) {
   return p;
 }
 
-// Steps of D positions for short cycles: a pass whose segments average at
-// most D positions computes no source positions past their ends (D = 8 over
-// 2-cycles of composed maps spent three quarters of its instructions there).
-template <typename Word, int D>
-void launch_cycle_short(const CycArgs& a, int variant, uint32_t blocks, hipStream_t stream) {
-  if (variant == 4)
-    hipLaunchKernelGGL((k_cycle<Word, D, 2>), dim3(blocks), dim3(256), 0, stream, a);
-  else if (variant == 5)
-    hipLaunchKernelGGL((k_cycle<Word, D, 3>), dim3(blocks), dim3(256), 0, stream, a);
-  else
-    hipLaunchKernelGGL((k_cycle<Word, D>), dim3(blocks), dim3(256), 0, stream, a);
-}
-
 template <typename Word>
-hipError_t launch_cycle_w(CycArgs a, int variant, uint32_t mean, hipStream_t stream) {
+hipError_t launch_cycle_w(CycArgs a, int variant, hipStream_t stream) {
   if (a.nslots) {
     const uint64_t words = a.B * a.nslots * (a.U / sizeof(Word));
     const uint64_t blocks = std::min<uint64_t>((words + 255) / 256, 256ull * 64);
     hipLaunchKernelGGL((k_cycle_save<Word>), dim3((uint32_t)blocks), dim3(256), 0, stream, a);
   }
   const uint64_t blocks = ((a.items << a.lane_log2) + 255) / 256;
-  if constexpr (sizeof(Word) == 16) {
-    if ((variant == 0 || variant == 4 || variant == 5) && mean && mean <= 4) {
-      if (mean <= 2) launch_cycle_short<Word, 2>(a, variant, (uint32_t)blocks, stream);
-      else launch_cycle_short<Word, 4>(a, variant, (uint32_t)blocks, stream);
-      return hipGetLastError();
-    }
-  }
   if (a.lane_log2 < 6 && variant >= 1 && variant <= 3)  // one item per wave only
     hipLaunchKernelGGL((k_cycle<Word, 8>), dim3((uint32_t)blocks), dim3(256), 0, stream, a);
   else if (variant == 1)
@@ -2088,10 +2068,11 @@ hipError_t prepare_cycle_args(const Op& op, char* data, char* scratch, int64_t s
 }
 
 // ---------------------------------------------------------------------------
-// Cycle following of cells that are not whole aligned 16-byte words
-// (k_cycle_u).  An item owns the cell-relative bytes [r0, r0 + n) of every
-// cell of its segment, r0 = g*G with G at most (lanes - 2) * 16 bytes and a
-// whole number of words, so items that share cells never touch each other's
+// Cycle following of cells that are not whole aligned 16-byte words, in
+// batches (a pass by itself runs k_cycle16).  An item owns the cell-relative
+// bytes [r0, r0 + n) of every cell of its segment, r0 = g*G with G at most
+// (lanes - 2) * 16 bytes and a whole number of words, so items that share
+// cells never touch each other's
 // bytes and every range starts and ends on a word.  At each position the item's
 // lanes cover the aligned 16-byte chunks of the destination's range (at
 // most lanes - 1 of them): lane l takes chunk X = (first chunk) + 16*l.
@@ -2373,11 +2354,6 @@ __device__ __forceinline__ void cycle_u_body(const CycArgs& a, const CycUArgs& u
   }
 }
 
-template <typename Word, typename Off, int D, int NM = kMaxCycleMaps>
-__global__ __launch_bounds__(256) void k_cycle_u(CycArgs a, CycUArgs u) {
-  cycle_u_body<Word, Off, D, NM>(a, u, (uint64_t)blockIdx.x * blockDim.x + threadIdx.x);
-}
-
 // Item geometry of the shifted cycle kernel for cells of w-byte words: fills
 // u and a.items.  Lanes per item: G <= (lanes - 2) * 16 cell bytes need at
 // most lanes - 1 destination chunks, so the last lane only hands its chunk
@@ -2403,69 +2379,20 @@ inline uint64_t cycu_threads(const CycArgs& a, const CycUArgs& u) {
   return (a.items + u.per_wave - 1) / u.per_wave * 64;
 }
 
-template <typename Word>
-hipError_t launch_cycle_u(CycArgs a, int depth, hipStream_t stream) {
-  if (a.nslots) {
-    const uint64_t words = a.B * a.nslots * (a.U / sizeof(Word));
-    const uint64_t blocks = std::min<uint64_t>((words + 255) / 256, 256ull * 64);
-    hipLaunchKernelGGL((k_cycle_save<Word>), dim3((uint32_t)blocks), dim3(256), 0, stream, a);
-  }
-  CycUArgs u;
-  const bool off32 = cycle_u_geometry(a, u, sizeof(Word));
-  const uint64_t blocks = (cycu_threads(a, u) + 255) / 256;
-  if (blocks >= (1ull << 31)) return hipErrorInvalidValue;
-  const dim3 grid((uint32_t)blocks), block(256);
-  if (off32) {
-    // passes of one or two composed maps (most) at the default depth: the
-    // kernel instantiated for two maps
-    if (depth == 4 && a.nmaps <= 2)
-      hipLaunchKernelGGL((k_cycle_u<Word, int32_t, 4, 2>), grid, block, 0, stream, a, u);
-    else if (depth == 4) hipLaunchKernelGGL((k_cycle_u<Word, int32_t, 4>), grid, block, 0, stream, a, u);
-    else if (depth == 6) hipLaunchKernelGGL((k_cycle_u<Word, int32_t, 6>), grid, block, 0, stream, a, u);
-    else hipLaunchKernelGGL((k_cycle_u<Word, int32_t, 8>), grid, block, 0, stream, a, u);
-  } else {
-    if (depth == 4) hipLaunchKernelGGL((k_cycle_u<Word, int64_t, 4>), grid, block, 0, stream, a, u);
-    else if (depth == 6) hipLaunchKernelGGL((k_cycle_u<Word, int64_t, 6>), grid, block, 0, stream, a, u);
-    else hipLaunchKernelGGL((k_cycle_u<Word, int64_t, 8>), grid, block, 0, stream, a, u);
-  }
-  return hipGetLastError();
-}
-
 hipError_t launch_cycle(const Op& op, char* data, char* scratch, int64_t scratch_bytes,
-                        int variant, int depth, hipStream_t stream, const void* table) {
+                        int variant, hipStream_t stream, const void* table) {
   CycArgs a;
   int64_t w = 1;
   bool empty = false;
   hipError_t e =
       prepare_cycle_args(op, data, scratch, scratch_bytes, &variant, a, &w, &empty, table);
   if (e != hipSuccess || empty) return e;
-  if (w < 16 && variant == 0) {  // cells that are not whole 16-byte words
-    switch (w) {
-      // cells of 8-byte words run the 4-byte kernel (95 instead of 112
-      // VGPRs: 5 waves per SIMD instead of 4); its edge pieces still include
-      // aligned 8-byte stores
-      case 8:
-      case 4: return launch_cycle_u<uint32_t>(a, depth, stream);
-      case 2: return launch_cycle_u<uint16_t>(a, depth, stream);
-      default: return launch_cycle_u<uint8_t>(a, depth, stream);
-    }
-  }
-  // cells of at least 512 bytes of 16-byte words: non-temporal loads and
-  // stores (variant 5), measured 1.7 % faster on 512-byte cells and 2-7 %
-  // on larger ones; smaller cells lose up to 70 % with them (neighbouring
-  // cells share cache lines that the hints evict).  Smaller cells in passes
-  // of at least 512 MiB: non-temporal stores only (variant 4), 2-6 % faster
-  // on 128-464-byte cells of 0.8-4 GB passes; a 231 MB pass, which the
-  // 256 MB last-level cache could hold, was 30 % slower with them
-  if (variant == 0 && w == 16 && a.U >= 512) variant = 5;
-  else if (variant == 0 && w == 16 && a.B * a.RCU >= (512ull << 20)) variant = 4;
-  const uint32_t mean = op.cyc->mean;
   switch (w) {
-    case 16: return launch_cycle_w<W16>(a, variant, mean, stream);
-    case 8: return launch_cycle_w<uint64_t>(a, variant, mean, stream);
-    case 4: return launch_cycle_w<uint32_t>(a, variant, mean, stream);
-    case 2: return launch_cycle_w<uint16_t>(a, variant, mean, stream);
-    default: return launch_cycle_w<uint8_t>(a, variant, mean, stream);
+    case 16: return launch_cycle_w<W16>(a, variant, stream);
+    case 8: return launch_cycle_w<uint64_t>(a, variant, stream);
+    case 4: return launch_cycle_w<uint32_t>(a, variant, stream);
+    case 2: return launch_cycle_w<uint16_t>(a, variant, stream);
+    default: return launch_cycle_w<uint8_t>(a, variant, stream);
   }
 }
 
@@ -3452,9 +3379,14 @@ hipError_t prepare_op(const Op& op) {
 
 hipError_t launch_op(const Op& op, char* data, char* scratch, int64_t scratch_bytes,
                      const LaunchCfg& cfg, hipStream_t stream, const void* table) {
+  if (op.kind == OP_CYCLE && cycle16_takes(op, cfg)) {
+    hipError_t e = hipSuccess;
+    if (op.cyc->segs.empty()) return e;  // fixed points only
+    if (!table && !(table = cycle_table_device(*op.cyc, &e))) return e;
+    return launch_cycle16(op, data, scratch, scratch_bytes, cfg, stream, table);
+  }
   if (op.kind == OP_CYCLE)
-    return launch_cycle(op, data, scratch, scratch_bytes, cfg.cycle_variant, cfg.cycle_u_depth, stream,
-                        table);
+    return launch_cycle(op, data, scratch, scratch_bytes, cfg.cycle_variant, stream, table);
   if (op.kind == OP_BLOCK) return launch_block(op, data, cfg, stream, table);
   if (op.kind == OP_SEGTILE) return launch_segtile(op, data, cfg, stream);
   if (op.kind == 0 || op.us <= 0 || op.U % op.us) return hipErrorInvalidValue;

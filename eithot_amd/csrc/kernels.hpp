@@ -22,7 +22,6 @@ struct LaunchCfg {
   int segtile_threads = 0;         // > 0: workgroup size of segmented tile passes
   int lds_threads_auto = 1;        // 1: tile/column/row workgroups sized for one load round
   int segtile_nt = 3;              // non-temporal segmented tile loads (bit 0) and stores (bit 1)
-  int cycle_u_depth = 4;           // positions in flight per item of the shifted cycle kernel
   int64_t min_groups = 1024;       // workgroups a pass's footprints spread over at least (fewer
                                    // footprints per workgroup below that); batched launches,
                                    // whose passes share the GPU, use 1
@@ -36,6 +35,12 @@ struct LaunchCfg {
 // table on first use.  Returns a hipError_t.
 hipError_t launch_op(const Op& op, char* data, char* scratch, int64_t scratch_bytes,
                      const LaunchCfg& cfg, hipStream_t stream, const void* table = nullptr);
+
+// Cycle passes over cells of at least 16 bytes (cycle.hip): whether they take
+// this op under cfg, and the launch; `table` is the op's device table.
+bool cycle16_takes(const Op& op, const LaunchCfg& cfg);
+hipError_t launch_cycle16(const Op& op, char* data, char* scratch, int64_t scratch_bytes,
+                          const LaunchCfg& cfg, hipStream_t stream, const void* table);
 
 // Uploads what an op needs on the current device before its first launch
 // (the cycle table of OP_CYCLE; nothing for other kinds).  Call before

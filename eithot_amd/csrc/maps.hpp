@@ -95,6 +95,20 @@ struct FD32 {
   EH_HD uint32_t mod(uint32_t x) const { return x - div(x) * d; }
 };
 
+// Division of x < 2^31 by d >= 2 in two instructions: with 2^(l-1) < d <= 2^l
+// and mul = floor(2^(31+l) / d) + 1 < 2^32, x * mul / 2^(31+l) exceeds x / d
+// by less than 2^31 / 2^(31+l) <= 1/d, so the floors agree.
+struct FD31 {
+  uint32_t mul = 0, s = 0;
+  void init(uint32_t d) {
+    uint32_t l = 1;
+    while (((uint64_t)1 << l) < d) ++l;
+    mul = (uint32_t)(((uint64_t)1 << (31 + l)) / d + 1);
+    s = l - 1;
+  }
+  EH_HD uint32_t div(uint32_t x) const { return mulhi32(x, mul) >> s; }
+};
+
 // Source cell of a digit permutation, stepped cell by cell.  A cell index
 // o has mixed-radix digits d_k (radix frad[k].d, fastest first) and its
 // source is sum d_k * stride[k]; step() moves to o + 1 with one add per

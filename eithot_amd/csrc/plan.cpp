@@ -599,6 +599,102 @@ const std::vector<int64_t>& divisors(int64_t x) {
 // Segment length of a cycle pass over B regions of N cells of U bytes:
 // short enough for about 32 Ki waves (one per segment and 1 KiB of cell),
 // long enough that the saved boundary cells and the table fit the budget.
+}  // namespace
+
+namespace {
+
+// A digit permutation of positions under construction: the value that the
+// maps applied so far give, as digits of the position in order of rising
+// weight.  Digit ids name the position's own digits; `ord` orders them.
+struct DigitBuild {
+  struct Dig {
+    int64_t radix;
+    int id;
+  };
+  std::vector<Dig> v;
+  std::vector<int> ord = {0};
+  int next = 1;
+  explicit DigitBuild(int64_t N) : v{{N, 0}} {}
+
+  // Splits a digit so that the first ones span exactly `span`; the index
+  // after them, or -1 when span does not divide the digits so.
+  int cut(int64_t span) {
+    int64_t n = 1;
+    for (size_t k = 0; k < v.size(); ++k) {
+      if (n == span) return (int)k;
+      if (span % n) return -1;
+      const int64_t a = span / n;
+      if (a < v[k].radix) {
+        if (v[k].radix % a) return -1;
+        const Dig hi = {v[k].radix / a, next++};
+        ord.insert(std::find(ord.begin(), ord.end(), v[k].id) + 1, hi.id);
+        v[k].radix = a;
+        v.insert(v.begin() + (long)k + 1, hi);
+        return (int)k + 1;
+      }
+      n *= v[k].radix;
+    }
+    return n == span ? (int)v.size() : -1;
+  }
+  // q = (j*R + i)*m + x of a block takes (i*C + j)*m + x
+  bool apply(const CycleMap& M) {
+    if (M.m < 1 || M.R < 1 || M.C < 1 || M.bc != M.m * M.R * M.C || cut(M.m) < 0 || cut(M.m * M.R) < 0 || cut(M.bc) < 0) return false;
+    const int x = cut(M.m), i = cut(M.m * M.R), j = cut(M.bc);
+    std::rotate(v.begin() + x, v.begin() + i, v.begin() + j);
+    return true;
+  }
+  // digits adjacent in both orders are one; false when too many are left
+  bool result(CycleDigits& d) const {
+    std::vector<int64_t> radix(next, 1), stride(next, 0);
+    int64_t w = 1;
+    for (const Dig& g : v) {
+      radix[g.id] = g.radix;
+      stride[g.id] = w;
+      w *= g.radix;
+    }
+    d = CycleDigits();
+    for (int id : ord) {
+      if (radix[id] == 1) continue;
+      if (d.n && (int64_t)d.stride[d.n - 1] * d.radix[d.n - 1] == stride[id]) {
+        d.radix[d.n - 1] *= (uint32_t)radix[id];
+        continue;
+      }
+      if (d.n == kMaxCycleDigits) return false;
+      d.radix[d.n] = (uint32_t)radix[id];
+      d.stride[d.n++] = (uint32_t)stride[id];
+    }
+    return true;
+  }
+};
+
+}  // namespace
+
+void cycle_digits(CycleTable& t, int64_t N) {
+  t.digits.clear();
+  if (N < 2 || N >= (1ll << 31)) return;
+  for (size_t k = t.maps.size(); k > 0;) {
+    DigitBuild b(N);
+    CycleDigits d;
+    bool any = false;
+    while (k > 0) {
+      DigitBuild c = b;
+      CycleDigits e;
+      if (!c.apply(t.maps[k - 1]) || !c.result(e)) break;
+      b = std::move(c);
+      d = e;
+      any = true;
+      --k;
+    }
+    if (!any) {  // a map that does not divide N: no digit form
+      t.digits.clear();
+      return;
+    }
+    t.digits.push_back(d);
+  }
+}
+
+namespace {
+
 std::shared_ptr<CycleTable> choose_cycle_table(const std::vector<CycleMap>& maps, int64_t N,
                                                int64_t B, int64_t U, int64_t budget,
                                                int64_t lmax0) {
@@ -632,6 +728,7 @@ std::shared_ptr<CycleTable> choose_cycle_table(const std::vector<CycleMap>& maps
     for (const CycleSeg& s : t->segs) sorted[at[group(s)]++] = s;
     t->segs.swap(sorted);
   }
+  cycle_digits(*t, N);
   return t;
 }
 

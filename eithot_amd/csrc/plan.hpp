@@ -92,6 +92,11 @@ struct CycleMap {
   int64_t bc, R, C, m;
 };
 constexpr int kMaxCycleMaps = 5;  // maps one cycle pass composes
+constexpr int kMaxCycleDigits = 8;  // digits of one digit permutation of positions
+struct CycleDigits {
+  int n = 0;
+  uint32_t radix[kMaxCycleDigits] = {0}, stride[kMaxCycleDigits] = {0};
+};
 struct CycleTable {
   int64_t lmax = 0;
   // maps applied in pass order; the pass's source of position p is
@@ -109,7 +114,32 @@ struct CycleTable {
   int64_t bytes() const { return (int64_t)(segs.size() * sizeof(CycleSeg) + slots.size() * 4); }
   // device copies (segs then slots), one per device id, made by the launcher
   DeviceCopies dev;
+  // The source as digit permutations, applied in order (cycle_digits): with
+  // p's mixed-radix digits d_k (radix[k], fastest first) each takes p to
+  // sum d_k * stride[k].  One for all maps where their factors divide each
+  // other's digits, one more from every map where they do not.
+  std::vector<CycleDigits> digits;
 };
+// Bytes of a cell (16 and more) that one item of a cycle pass moves, 16 to a
+// lane: the whole cell up to 1 KiB, or whole 128-byte lines of it where that
+// leaves fewer lanes of the waves idle (by a tenth at least: 1408-byte cells
+// as 512 + 512 + 384 bytes in 32 lanes each; cut in two halves of 44 lanes,
+// one to a wave, they took 91 us instead of 75 per 212 MB).  A cell's last
+// group keeps 16 bytes and more.
+inline uint32_t cycle_cell_group(uint32_t U) {
+  auto ends = [&](uint32_t G) { return G >= U || U % G == 0 || U % G >= 16; };
+  auto used = [&](uint32_t G) {  // share of lanes at work
+    const uint32_t lanes = (G + 15) / 16, groups = (U + G - 1) / G;
+    return (double)U / 16 * (64 / lanes) / (64.0 * groups);
+  };
+  uint32_t best = U <= 1024 ? U : 1024;
+  while (!ends(best)) best -= 16;
+  for (uint32_t G : {512u, 256u, 128u})
+    if (G < U && ends(G) && used(G) > 1.1 * used(best)) best = G;
+  return best;
+}
+// Fills t.digits from its maps over N < 2^31 positions.
+void cycle_digits(CycleTable& t, int64_t N);
 // Builds the table (fixed points are skipped).  R*C must be below 2^32.
 std::shared_ptr<CycleTable> build_cycle_table(int64_t R, int64_t C, int64_t lmax);
 // Same over the composition of several cell maps on N cells (N < 2^32).
@@ -234,7 +264,7 @@ struct Tuning {
   int64_t segtile_nt = 3;
   int64_t lower_mask = LOWER_ALL;
   int64_t hold_floor = 64ll << 20;  // device bytes the library may keep whatever alpha allows
-  int64_t cycle_u_depth = 4;        // positions in flight per item of the shifted cycle kernel (4, 6, 8)
+  int64_t cycle_u_depth = 4;        // accepted (4, 6, 8), no effect
   int64_t min_groups = 1024;        // workgroups a single-launch pass spreads its footprints over
   int64_t whole = 1;                // whole-permutation passes (whole.hpp) where they fit
   bool plain = true;   // every knob of the passes has its default value

@@ -212,16 +212,15 @@ int eithot_plan_segments(const int64_t* dims, const int* perm, int order, size_t
  *   "block_pad"      fused blocks pad their LDS copy where a bank-conflict
  *                    model says it pays (1) or never (0)
  *   "cycle_variant"  cycle-following kernel shape (0..7; 1..3 only for cells of
- *                    at least 64 words).  0 (default) picks: shifted 16-byte
- *                    chunks for cells that are not whole 16-byte words,
- *                    non-temporal loads and stores (as 5) for cells of at
- *                    least 512 bytes, non-temporal stores (as 4) for
- *                    smaller 16-byte-word cells in passes of at least
- *                    512 MiB, else plain 16-byte words
+ *                    at least 64 words).  0 (default): 16 bytes per lane
+ *                    whatever the cell's size and address, non-temporal
+ *                    loads and stores for cells of at least 512 bytes in
+ *                    whole aligned 16-byte words, non-temporal stores for
+ *                    smaller ones in passes of at least 512 MiB
  *   "cycle_lmax"     > 0: cycle segments of at most this many positions
  *                    (0: chosen per pass)
- *   "cycle_u_depth"  positions in flight per item when cycle following moves
- *                    cells that are not whole 16-byte words (4 default, 6, 8)
+ *   "cycle_u_depth"  4 (default), 6 or 8: once the positions in flight of cells
+ *                    that are not whole 16-byte words; accepted, no effect
  *   "min_groups"     workgroups a pass launched on its own spreads its LDS
  *                    footprints over, at least (1024; 1..2^20); batched
  *                    launches pack footprints to the LDS target instead
