@@ -290,14 +290,15 @@ WholePass plan_whole(const int64_t* dims, const int* perm1, int rank, size_t ele
     uint32_t per;
   };
   constexpr Step kSteps[] = {{6, 256, 1},  {10, 256, 1},  {19, 256, 1},  {38, 256, 1},
-                             {78, 512, 1}, {156, 1024, 1}, {156, 1024, 2}};
+                             {78, 512, 2}, {156, 1024, 2}};
   // resident: tiles as small as keeps the workgroups of a small tensor below
   // three per CU (77 KB: 17 -> 9.5 us, 4.4 MB: 33 -> 13 us, 1 MB of bytes:
   // 59 -> 10 us against the ordinary passes; meeting costs 2 to 5 us), and
-  // 64 KiB tiles, two workgroups per CU, for larger ones and batches
-  // (210 MB in regions of 3.6 MB: 158 -> 114 us; 32 KiB tiles 117, 128 KiB
-  // 132).  Where a region does not fit so, workgroups hold a second tile in
-  // registers.  A region takes at most half of the workgroups the chip holds, so
+  // 64 KiB tiles, two workgroups per CU and a second tile of each in
+  // registers, for larger ones and batches (210 MB in regions of 3.6 MB:
+  // 158 -> 100 us; one tile each 114, 32 KiB tiles 99, but 38 instead of 43 us
+  // for 52 MB of bytes and 121 instead of 117 for 236 MB; 128 KiB 130).  A
+  // region takes at most half of the workgroups the chip holds, so
   // that two processes can always run theirs.
   if (c.B <= (int64_t)kWholeRegions) {
     std::vector<int> cls(r);
