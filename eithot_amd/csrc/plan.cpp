@@ -763,8 +763,9 @@ inline double staged_tile_cost(int64_t R, int64_t U, int64_t us) {
   return us < 16 && !packs ? 3.0 * c : c;
 }
 
-// Cycle-following moves whole cells (of at least cycle_min_cell bytes), one
-// read and one write each; smaller cells waste HBM bursts.
+// Cycle-following moves whole cells, one read and one write each; cells of
+// less than cycle_min_cell bytes waste HBM bursts and take it where the other
+// lowerings are slower still.
 constexpr uint64_t kCycleMaxCells = 1ull << 26;
 // Composite cycle tables of two-pass regroup plans may span more cells: the
 // plan replaces a whole pass of a large tensor (host walk: about 40 ns per
@@ -780,7 +781,27 @@ constexpr double kCostCycleShift = 1.35;
 thread_local bool g_cycle_word_cost = true;  // off: every cell width costs the same
 thread_local bool g_cycle_cell_pref = false;  // on: larger cells cost less
 thread_local bool g_cycle_shift = true;       // narrow cells move in shifted 16-byte chunks
+thread_local int64_t g_cycle_min_cell = 0;    // cells below cost as small ones
+thread_local bool g_cycle_small = false;      // cycle passes may move small cells
+// Cycle passes over cells of 16 bytes to a line (k_cycle16) fetch whole lines
+// for parts of them.  In the cost unit (5.2 TB/s), from 314 MB transposes of
+// 14 and 1213 rows: 64 bytes 196-204 us, 72-124 bytes 201-264, 32-50 bytes
+// 357-456, 20-24 bytes 607-671, 16 bytes 887; from 64 bytes 0.15 more, against
+// plans that would only tie.
+constexpr uint64_t kCycleMaxSmallCells = 1ull << 23;  // planned in 0.2-0.35 s
+inline double small_cycle_cost(int64_t U) {
+  if (U >= 64) return U % 64 ? 2.05 : 1.8;
+  return U >= 32 ? 3.3 : U > 16 ? 5.5 : 7.4;
+}
+// What a column or row pass of such cells takes beyond cat_pass_cost, in the
+// same unit.  Above, a pair took 580-1000 us with a staged pass, and 42 MB
+// 45-120 us in LDS (cycles: 29-57 from 32 bytes, 72-99 below) and 166-360 us
+// in slices under 16 bytes.
+inline double small_cat_extra(int64_t us, bool staged) {
+  return us < 16 ? 3.0 : staged ? 2.7 : 1.0;
+}
 inline double cycle_cost(int64_t U) {
+  if (U < g_cycle_min_cell) return small_cycle_cost(U);
   const int64_t w = pow2_factor(U, 16);
   if (!g_cycle_word_cost) return kCostCycle;
   if (w < 16) return g_cycle_shift ? kCostCycleShift : w == 8 ? 2.0 : w == 4 ? 4.0 : 6.0;
@@ -880,6 +901,19 @@ struct Lowerer {
           ch.cost = c1 + c2 + kCostSplit;
         }
       }
+    }
+    // cells of 16 bytes to a line along cycles too, where all of the above is
+    // slower; the parents' choices stay on the costs above, and what nothing
+    // above can lower stays so (batches, whose cycle kernel moves narrow
+    // words, don't)
+    if ((mask & LOWER_CYCLE) && g_cycle_small && ch.how != HOW_NONE && U >= 16 &&
+        U < prof.cycle_min_cell && (uint64_t)R * (uint64_t)C <= kCycleMaxSmallCells &&
+        cycle_cost(U) < ch.cost + (ch.how == HOW_CAT
+                                       ? small_cat_extra(cp.row_us, cp.row_staged) +
+                                             (cp.npass - 1) * small_cat_extra(cp.col_us, cp.col_staged)
+                                       : 0.0)) {
+      ch.how = HOW_CYCLE;
+      ch.cost = std::min(ch.cost, cycle_cost(U));
     }
     memo[key] = ch;
     return ch;
@@ -1224,10 +1258,9 @@ std::shared_ptr<BlockTable> compose_tiles(const std::vector<int64_t>& parts, int
   return t;
 }
 
-// Consecutive passes that permute whole cells of at least cycle_min_cell
-// bytes over the same bytes (cycle passes and whole-unit tiles) compose into
-// one cycle pass over cells of their common size, when at least one of them
-// is a cycle pass.
+// Consecutive passes that permute whole cells of at least 16 bytes over the
+// same bytes (cycle passes and whole-unit tiles) compose into one cycle pass
+// over cells of their common size, when at least one of them is a cycle pass.
 void fuse_cycles(std::vector<Op>& ops, const DeviceProfile& prof) {
   if (prof.cycle_min_cell <= 0) return;
   auto cellperm = [&](const Op& o) {
@@ -1244,14 +1277,17 @@ void fuse_cycles(std::vector<Op>& ops, const DeviceProfile& prof) {
     while (j < ops.size() && cellperm(ops[j]) && maps_n + nmaps(ops[j]) <= 4 &&
            ops[j].base == ops[i].base && ops[j].bytes() == ops[i].bytes()) {
       const int64_t g2 = gcd64(g, ops[j].U);
-      if (g2 < prof.cycle_min_cell || ops[j].bytes() / (uint64_t)g2 > kCycleMaxCells) break;
+      if (g2 < (g_cycle_small ? std::min<int64_t>(16, prof.cycle_min_cell) : prof.cycle_min_cell) ||
+          ops[j].bytes() / (uint64_t)g2 >
+              (g2 < prof.cycle_min_cell ? kCycleMaxSmallCells : kCycleMaxCells))
+        break;
       g = g2;
       cycles += ops[j].kind == OP_CYCLE;
       maps_n += nmaps(ops[j]);
       ++j;
     }
     // composing must not cost more than the parts (a smaller common cell
-    // can force narrower words)
+    // can fill its lines less)
     while (j - i >= 2) {
       double parts = 0;
       int64_t gg = 0;
@@ -1314,6 +1350,16 @@ double plan_cost(const Plan& plan) {
       case OP_SEGTILE: c += segtile_cost(o); break;
     }
   }
+  return c;
+}
+
+// The same with the column and row passes that small cells' cycles replace at
+// what they take.
+double small_cell_cost(const Plan& plan) {
+  double c = plan_cost(plan);
+  for (const Op& o : plan.ops)
+    if ((o.kind == OP_COL || o.kind == OP_ROW) && o.U >= 16 && o.U < g_cycle_min_cell)
+      c += small_cat_extra(o.us, o.staged != 0);
   return c;
 }
 
@@ -1862,14 +1908,14 @@ static void finalize_plan(Plan& plan, double alpha, int64_t reserve, const Devic
 
 static int make_plan_search(const int64_t* dims_in, const int* perm1, int rank, size_t elem,
                             int n_sub, double alpha, const DeviceProfile& prof, int reorder,
-                            Plan& plan);
+                            Plan& plan, bool small);
 
 // Planning allocates host tables that can be large (a cycle table spans up
 // to 2^28 cells); running out of host memory is reported, not thrown.
 int make_plan(const int64_t* dims_in, const int* perm1, int rank, size_t elem, int n_sub,
               double alpha, const DeviceProfile& prof, int reorder, Plan& plan) {
   try {
-    return make_plan_search(dims_in, perm1, rank, elem, n_sub, alpha, prof, reorder, plan);
+    return make_plan_search(dims_in, perm1, rank, elem, n_sub, alpha, prof, reorder, plan, true);
   } catch (const std::bad_alloc&) {
     plan = Plan();
     return EITHOT_ERR_NOMEM;
@@ -1881,10 +1927,11 @@ int make_plan(const int64_t* dims_in, const int* perm1, int rank, size_t elem, i
 
 static int make_plan_search(const int64_t* dims_in, const int* perm1, int rank, size_t elem,
                             int n_sub, double alpha, const DeviceProfile& prof, int reorder,
-                            Plan& plan) {
+                            Plan& plan, bool small) {
   g_cycle_word_cost = prof.cycle_word_cost != 0;
   g_cycle_cell_pref = prof.cycle_cell_pref != 0;
   g_cycle_shift = prof.cycle_shift != 0;
+  g_cycle_min_cell = prof.cycle_min_cell;
   // Search: decomposer order (pre/post, or the one asked for) x how hard
   // staged passes are avoided; cycle passes that later compose with their
   // neighbours make a split lowering cheaper than a staged one, which only
@@ -1935,53 +1982,74 @@ static int make_plan_search(const int64_t* dims_in, const int* perm1, int rank, 
   Regroup rg;
   const bool regroup = vol_ok && !partition && reorder == 0 && prof.regroup &&
                        rg.canonical(dims_in, perm1, rank, elem) && rg.q.size() >= 3;
-  for (double mult : {1.0, 3.0}) {
-    DeviceProfile p2 = prof;
-    p2.staged_mult = mult;
-    Lowerer shared(p2, budget0);
-    for (int o : orders) {
-      Plan q;
-      const int r =
-          make_plan_impl(dims_in, perm1, rank, elem, n_sub, alpha, p2, o, 0, q, &shared);
-      if (r) {
-        if (rc) rc = r;
-        continue;
+  auto search = [&] {
+    for (double mult : {1.0, 3.0}) {
+      DeviceProfile p2 = prof;
+      p2.staged_mult = mult;
+      Lowerer shared(p2, budget0);
+      for (int o : orders) {
+        Plan q;
+        const int r =
+            make_plan_impl(dims_in, perm1, rank, elem, n_sub, alpha, p2, o, 0, q, &shared);
+        if (r) {
+          if (rc) rc = r;
+          continue;
+        }
+        const double c = plan_cost(q);
+        if (rc || c < best_cost - 1e-9) {
+          best_cost = c;
+          best_order = o;
+          best_mult = mult;
+          plan = std::move(q);
+        }
+        rc = EITHOT_OK;
       }
-      const double c = plan_cost(q);
-      if (rc || c < best_cost - 1e-9) {
-        best_cost = c;
-        best_order = o;
-        best_mult = mult;
-        plan = std::move(q);
-      }
-      rc = EITHOT_OK;
-    }
-    if (!regroup || (rc && rc != EITHOT_ERR_ALPHA)) continue;
-    const int n = (int)rg.q.size();
-    for (int i = 1; i < n && i <= 6; ++i)
-      for (int j = 1; i + j <= n && j <= 6; ++j)
-        for (bool zo : {false, true}) {
-          if (zo && i + j == n) continue;  // no Z: both orders agree
-          for (int form = 0; form < 5; ++form) {
-            Plan q;
-            const bool ok =
-                form == 0   ? regroup_plan(rg, i, j, zo, elem, shared, p2, q)
-                : form <= 2 ? regroup2_plan(rg, i, j, zo, form == 1, elem, p2, q)
-                            : regroup2_split(rg, i, j, zo, form == 3, elem, p2,
-                                             rc ? 1e300 : best_cost, q);
-            if (!ok) continue;
-            q.tensor_bytes = vol * elem;
-            const double c = plan_cost(q);
-            if (rc || c < best_cost - 1e-9) {
-              best_cost = c;
-              best_mult = mult;
-              plan = std::move(q);
-              rc = EITHOT_OK;
+      if (!regroup || (rc && rc != EITHOT_ERR_ALPHA)) continue;
+      const int n = (int)rg.q.size();
+      for (int i = 1; i < n && i <= 6; ++i)
+        for (int j = 1; i + j <= n && j <= 6; ++j)
+          for (bool zo : {false, true}) {
+            if (zo && i + j == n) continue;  // no Z: both orders agree
+            for (int form = 0; form < 5; ++form) {
+              Plan q;
+              const bool ok =
+                  form == 0   ? regroup_plan(rg, i, j, zo, elem, shared, p2, q)
+                  : form <= 2 ? regroup2_plan(rg, i, j, zo, form == 1, elem, p2, q)
+                              : regroup2_split(rg, i, j, zo, form == 3, elem, p2,
+                                               rc ? 1e300 : best_cost, q);
+              if (!ok) continue;
+              q.tensor_bytes = vol * elem;
+              const double c = plan_cost(q);
+              if (rc || c < best_cost - 1e-9) {
+                best_cost = c;
+                best_mult = mult;
+                plan = std::move(q);
+                rc = EITHOT_OK;
+              }
             }
           }
-        }
-  }
+    }
+  };
+  g_cycle_small = false;
+  search();
   if (rc) return rc;
+  // again with cycle passes of small cells, kept where they cost less
+  if (small && g_cycle_shift) {
+    Plan first = std::move(plan);
+    const int order1 = best_order;
+    const double mult1 = best_mult;
+    g_cycle_small = true;
+    rc = EITHOT_ERR_INVALID;
+    best_cost = 1e300;
+    plan = Plan();
+    search();
+    if (rc || small_cell_cost(plan) >= small_cell_cost(first) - 1e-9) {
+      plan = std::move(first);
+      best_order = order1;
+      best_mult = mult1;
+      g_cycle_small = false;
+    }
+  }
   DeviceProfile pb = prof;
   pb.staged_mult = best_mult;
   finalize_plan(plan, alpha, 0, pb);
@@ -1993,6 +2061,13 @@ static int make_plan_search(const int64_t* dims_in, const int* perm1, int rank, 
   const int64_t budget = (int64_t)(alpha * (double)plan.tensor_bytes);
   auto extra = [](const Plan& p) { return p.scratch_bytes + p.table_bytes; };
   if (extra(plan) <= budget) return EITHOT_OK;
+  // small cells make longer tables: first without them
+  if (small && std::any_of(plan.ops.begin(), plan.ops.end(), [&](const Op& o) {
+        return o.kind == OP_CYCLE && o.U < prof.cycle_min_cell;
+      })) {
+    plan = Plan();
+    return make_plan_search(dims_in, perm1, rank, elem, n_sub, alpha, prof, reorder, plan, false);
+  }
   Plan best = plan;
   for (int attempt = 0; attempt < 3; ++attempt) {
     int64_t reserve = 0;
