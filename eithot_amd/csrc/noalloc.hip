@@ -50,6 +50,36 @@ eithot::LruCache<eithot::Plan>& plans() {
   return *c;
 }
 
+size_t align_up(size_t n) { return (n + kAlign - 1) / kAlign * kAlign; }
+
+// Device table bytes of one op (0 when it reads none), laid out as the
+// launcher uploads them.
+size_t table_bytes(const eithot::Op& op) {
+  if (op.kind == eithot::OP_CYCLE && op.cyc && !op.cyc->segs.empty())
+    return op.cyc->segs.size() * sizeof(eithot::CycleSeg) + op.cyc->slots.size() * 4;
+  if (op.kind == eithot::OP_BLOCK && op.blk && !op.blk->ndig)
+    return op.blk->src.size() * (op.blk->cells <= 65536 ? 2 : 4);
+  return 0;
+}
+
+// Offsets of the pass tables (each on a 256-byte boundary), and of the
+// scratch after them.
+size_t layout(const eithot::Plan& plan, std::vector<size_t>& toff) {
+  size_t used = 0;
+  toff.assign(plan.ops.size(), 0);
+  for (size_t i = 0; i < plan.ops.size(); ++i) {
+    const size_t tb = table_bytes(plan.ops[i]);
+    if (!tb) continue;
+    toff[i] = used;
+    used += align_up(tb);
+  }
+  return used;
+}
+size_t needs(const eithot::Plan& plan) {
+  std::vector<size_t> toff;
+  return layout(plan, toff) + align_up((size_t)std::max<int64_t>(plan.scratch_bytes, 0));
+}
+
 eithot::PlanPtr plan_noalloc(const eithot::Device* d, const int64_t* dims, const int* perm,
                              int order, size_t elem, int n_sub, double alpha, int* rc) {
   const std::string key = std::to_string(d->id) + "@" +
@@ -61,27 +91,20 @@ eithot::PlanPtr plan_noalloc(const eithot::Device* d, const int64_t* dims, const
       return p;
     }
   }
-  const eithot::DeviceProfile pr = d->profile();
+  eithot::DeviceProfile pr = d->profile();
   auto p = std::make_shared<eithot::Plan>();
   *rc = eithot::make_plan(dims, perm, order, elem, n_sub, alpha, pr, pr.reorder, *p);
+  if (*rc == EITHOT_OK && p->small_cells && needs(*p) > kNoAllocBytes) {
+    pr.cycle_small = 0;  // their tables don't fit: the plan without them may
+    p = std::make_shared<eithot::Plan>();
+    *rc = eithot::make_plan(dims, perm, order, elem, n_sub, alpha, pr, pr.reorder, *p);
+  }
   if (*rc != EITHOT_OK) return nullptr;
   std::vector<eithot::PlanPtr> evicted;
   std::lock_guard<std::mutex> lk(g_plan_mu);
   if (eithot::PlanPtr q = plans().get(key)) return q;
   evicted = plans().put(key, p, (uint64_t)std::max<int64_t>(p->table_bytes, 0));
   return p;
-}
-
-size_t align_up(size_t n) { return (n + kAlign - 1) / kAlign * kAlign; }
-
-// Device table bytes of one op (0 when it reads none), laid out as the
-// launcher uploads them.
-size_t table_bytes(const eithot::Op& op) {
-  if (op.kind == eithot::OP_CYCLE && op.cyc && !op.cyc->segs.empty())
-    return op.cyc->segs.size() * sizeof(eithot::CycleSeg) + op.cyc->slots.size() * 4;
-  if (op.kind == eithot::OP_BLOCK && op.blk && !op.blk->ndig)
-    return op.blk->src.size() * (op.blk->cells <= 65536 ? 2 : 4);
-  return 0;
 }
 
 }  // namespace
@@ -112,17 +135,8 @@ extern "C" int eithot_transpose_noalloc(void* dev, const int64_t* dims, const in
   lk.unlock();
   PlanPtr plan = plan_noalloc(d, dims, perm, order, elem_bytes, n_sub, alpha, &rc);
   if (!plan) return fail(rc, "planning failed (%d)", rc);
-  // layout: the pass tables (each on a 256-byte boundary), then the scratch
-  std::vector<size_t> toff(plan->ops.size(), 0);
-  size_t used = 0;
-  for (size_t i = 0; i < plan->ops.size(); ++i) {
-    const size_t tb = table_bytes(plan->ops[i]);
-    if (!tb) continue;
-    toff[i] = used;
-    used += align_up(tb);
-  }
-  const size_t scratch_off = used;
-  used += align_up((size_t)std::max<int64_t>(plan->scratch_bytes, 0));
+  std::vector<size_t> toff;
+  const size_t scratch_off = layout(*plan, toff), used = needs(*plan);
   if (used > kNoAllocBytes)
     return fail(EITHOT_ERR_NOMEM,
                 "the plan needs %zu bytes of scratch and pass tables; the static scratch of "

@@ -1915,7 +1915,8 @@ static int make_plan_search(const int64_t* dims_in, const int* perm1, int rank, 
 int make_plan(const int64_t* dims_in, const int* perm1, int rank, size_t elem, int n_sub,
               double alpha, const DeviceProfile& prof, int reorder, Plan& plan) {
   try {
-    return make_plan_search(dims_in, perm1, rank, elem, n_sub, alpha, prof, reorder, plan, true);
+    return make_plan_search(dims_in, perm1, rank, elem, n_sub, alpha, prof, reorder, plan,
+                            prof.cycle_small && prof.regroup);
   } catch (const std::bad_alloc&) {
     plan = Plan();
     return EITHOT_ERR_NOMEM;
@@ -2053,6 +2054,9 @@ static int make_plan_search(const int64_t* dims_in, const int* perm1, int rank, 
   DeviceProfile pb = prof;
   pb.staged_mult = best_mult;
   finalize_plan(plan, alpha, 0, pb);
+  plan.small_cells = std::any_of(plan.ops.begin(), plan.ops.end(), [&](const Op& o) {
+    return o.kind == OP_CYCLE && o.U < prof.cycle_min_cell;
+  });
   if (plan.table_bytes == 0) return EITHOT_OK;
   // The pass tables count as extra memory too.  When they push the plan
   // over its budget: plan again with their bytes kept back from the
@@ -2062,9 +2066,7 @@ static int make_plan_search(const int64_t* dims_in, const int* perm1, int rank, 
   auto extra = [](const Plan& p) { return p.scratch_bytes + p.table_bytes; };
   if (extra(plan) <= budget) return EITHOT_OK;
   // small cells make longer tables: first without them
-  if (small && std::any_of(plan.ops.begin(), plan.ops.end(), [&](const Op& o) {
-        return o.kind == OP_CYCLE && o.U < prof.cycle_min_cell;
-      })) {
+  if (plan.small_cells) {
     plan = Plan();
     return make_plan_search(dims_in, perm1, rank, elem, n_sub, alpha, prof, reorder, plan, false);
   }

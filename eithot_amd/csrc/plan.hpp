@@ -234,6 +234,8 @@ struct DeviceProfile {
   int64_t cycle_cell_pref = 0;    // 1: cycle passes of larger cells cost less
   int64_t lower_mask = LOWER_ALL; // lowering options the planner may use
   int whole = 1;                  // one whole-permutation pass where it fits (whole.hpp)
+  int cycle_small = 1;            // cycle passes may move cells of 16 bytes to cycle_min_cell
+                                  // (with regroup, whose knob stands for the wider search)
   int cycle_shift = 1;            // cycle passes of narrow cells run the shifted 16-byte
                                   // kernel (0: word by word, as in batched launches)
   double staged_mult = 1.0;       // planner-internal: weight of staged passes in the search
@@ -287,6 +289,7 @@ struct Plan {
   int64_t scratch_bytes = 0;  // device scratch the plan needs (0 if all LDS)
   int64_t table_bytes = 0;    // device cycle tables of its OP_CYCLE passes
   uint64_t tensor_bytes = 0;
+  bool small_cells = false;   // has cycle passes of cells under the profile's cycle_min_cell
   std::string describe() const;
   // Bytes of this plan's pass tables that are resident on device `dev`.
   int64_t device_table_bytes(int dev) const;

@@ -127,9 +127,11 @@ static bool only_pass_weak(const Plan& p) {
 }
 
 PlanPtr Device::plan_for(const int64_t* dims, const int* perm1, int rank, size_t elem, int n_sub,
-                         double alpha, int* rc) {
-  const DeviceProfile pr = profile();
-  const std::string key = plan_key(dims, perm1, rank, elem, n_sub, alpha);
+                         double alpha, int* rc, bool small) {
+  DeviceProfile pr = profile();
+  pr.cycle_small = small;
+  std::string key = plan_key(dims, perm1, rank, elem, n_sub, alpha);
+  if (!small) key += "|large cells";
   {
     std::lock_guard<std::mutex> lk(mu);
     if (PlanPtr p = plans.get(key)) {
@@ -518,6 +520,23 @@ static int transpose_impl(void* dev, const int64_t* dims, const int* perm, int o
     return rc;
   }
   if ((rc = d->whole_status())) return rc;
+  // small cells' passes need tables where others need none: a captured call
+  // without an earlier one to upload them takes the others
+  if (plan->small_cells && stream_captured(stream)) {
+    bool ready;
+    {
+      std::lock_guard<std::mutex> lk(d->enqueue_mu);
+      ready = d->arena_bytes >= plan->scratch_bytes &&
+              std::all_of(plan->ops.begin(), plan->ops.end(), [&](const Op& o) {
+                return !((o.cyc && !o.cyc->segs.empty() && !o.cyc->dev.has(d->id)) ||
+                         (o.blk && !o.blk->ndig && !o.blk->dev.has(d->id)));
+              });
+    }
+    if (!ready && !(plan = d->plan_for(dims, perm, order, elem, n_sub, alpha, &rc, false))) {
+      if (!g_err.size()) fail(rc, "planning failed (%d)", rc);
+      return rc;
+    }
+  }
   {
     std::lock_guard<std::mutex> lk(d->enqueue_mu);
     const bool whole = d->takes_whole_locked(*plan, stream);

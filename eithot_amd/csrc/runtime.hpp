@@ -53,9 +53,10 @@ struct Device {
 
   // The cached plan for these arguments, planned on first sight (outside
   // the cache lock).  The caller's reference keeps the plan alive even if
-  // the cache evicts it.
+  // the cache evicts it.  small false: without cycle passes of small cells,
+  // for callers that cannot give their tables and boundary cells a place.
   PlanPtr plan_for(const int64_t* dims, const int* perm1, int rank, size_t elem, int n_sub,
-                   double alpha, int* rc);
+                   double alpha, int* rc, bool small = true);
   // hardware profile / launch configuration with the tuning knobs applied
   DeviceProfile profile() const;
   LaunchCfg launch_cfg() const;

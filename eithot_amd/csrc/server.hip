@@ -225,6 +225,9 @@ int64_t eithot_server_submit(eithot_server* s, void* dev, const int64_t* dims, c
   int rc = validate(dev, dims, perm, order, elem_bytes);
   if (rc) return rc;
   PlanPtr plan = s->dev->plan_for(dims, perm, order, elem_bytes, 1, s->alpha, &rc);
+  // small cells' boundary slots don't fit: the plan without them may
+  if (plan && plan->small_cells && !s->pool.fits(plan->scratch_bytes))
+    plan = s->dev->plan_for(dims, perm, order, elem_bytes, 1, s->alpha, &rc, false);
   if (!plan) return rc ? rc : fail(EITHOT_ERR_INVALID, "planning failed");
   if (!s->pool.fits(plan->scratch_bytes))
     return fail(EITHOT_ERR_ALPHA, "request needs %lld scratch bytes, pool holds %lld",

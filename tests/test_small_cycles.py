@@ -75,3 +75,65 @@ def test_device(torch_cuda, dims, perm, elem):
             assert not out[:lead].any() and not out[lead + n:].any()
     finally:
         E.set_tuning("whole", whole)
+
+
+# a plan without tables or scratch before; with small cells it has both
+LIMITED = ([31, 279, 1213], [1, 3, 2], 4)
+
+
+@pytest.mark.gpu
+def test_captured_first_and_pool_too_small(torch_cuda):
+    # what needed neither a table nor scratch before still runs where neither
+    # has a place: captured on its first call, and served without a pool
+    torch = torch_cuda
+    dims, perm, elem = LIMITED
+    rng = np.random.default_rng(5)
+    n = int(np.prod(dims)) * elem
+    a = rng.integers(0, 256, n, dtype=np.uint8)
+    want = O.permute(a, dims, [p - 1 for p in perm], elem=elem).view(np.uint8).reshape(-1)
+    src = torch.from_numpy(a).cuda()
+    buf = src.clone()
+    ops, scratch = E.plan_describe(dims, perm, elem)
+    assert small_cells(ops) and scratch > 256
+    old = E.set_tuning("whole", 0)
+    try:
+        E.transpose_ptr(src.clone().data_ptr(), [64, 64], [2, 1], 4)  # the library is set up
+        side, graph = torch.cuda.Stream(), torch.cuda.CUDAGraph()
+        print("small cells: first call captured", flush=True)
+        with torch.cuda.stream(side):
+            graph.capture_begin(capture_error_mode="thread_local")
+            try:
+                E.transpose_ptr(buf.data_ptr(), dims, perm, elem, stream=side.cuda_stream)
+            finally:
+                graph.capture_end()
+        for _ in range(3):
+            buf.copy_(src)
+            torch.cuda.synchronize()
+            graph.replay()
+            torch.cuda.synchronize()
+            assert np.array_equal(buf.cpu().numpy(), want)
+        buf.copy_(src)
+        torch.cuda.synchronize()
+        print("small cells: served without a pool", flush=True)
+        server = E.Server(0)
+        server.submit(buf.data_ptr(), dims, perm, elem)
+        server.drain()
+        torch.cuda.synchronize()
+        assert np.array_equal(buf.cpu().numpy(), want)
+        # and with a call before, captured on the passes of that call
+        E.transpose_ptr(src.clone().data_ptr(), dims, perm, elem)
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.stream(side):
+            graph.capture_begin(capture_error_mode="thread_local")
+            try:
+                E.transpose_ptr(buf.data_ptr(), dims, perm, elem, stream=side.cuda_stream)
+            finally:
+                graph.capture_end()
+        for _ in range(3):
+            buf.copy_(src)
+            torch.cuda.synchronize()
+            graph.replay()
+            torch.cuda.synchronize()
+            assert np.array_equal(buf.cpu().numpy(), want)
+    finally:
+        E.set_tuning("whole", old)
