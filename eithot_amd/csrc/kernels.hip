@@ -2490,6 +2490,12 @@ struct BlkArgs {
   // their source offsets every P chunks (P * 16 = lcm(F, 16) bytes, a
   // multiple of the pad interval); 0: off
   uint32_t P;
+  // strided pattern stores (cells of one 1- or 2-byte word, fastest output
+  // digit under a chunk's V words): Q cells are the shortest product of leading output
+  // digits that spans a chunk, PQ chunks (PQ * V = lcm(Q, V)) their pattern;
+  // 0: off
+  uint32_t Q, PQ;
+  FD32 fQ, fnQ;  // Q, n / Q
 };
 
 // source cell of output cell o: digit form (at most ND digits), or the
@@ -2522,6 +2528,41 @@ __device__ __forceinline__ uint32_t blk_lds(const BlkArgs& a, uint32_t k, uint32
   return k * a.Fl + lds_off(x, a.pad);
 }
 
+// Chunks of V one-word cells whose fastest output digits are short: a thread
+// that strides the chunks by a multiple of PQ meets every chunk at the same
+// place `rel` of its period of Q cells, so the sources of its words relative
+// to their period are computed once, and a chunk takes the source of its
+// first period and, from its cell k1, of the next one.  The digit odometer
+// this replaces took about 20 instructions per word: 217 MB of bytes in
+// blocks of (3, 2, 181, 57) read out as (2, 3, 57, 181) 283 -> 192 us, 114 MB
+// in blocks of (601, 7, 3) as (3, 7, 601) 183 -> 88, 246 MB of 2-byte cells
+// in blocks of (2048, 2, 2, 3) as (2, 2, 2048, 3) 172 -> 132.  4-byte cells
+// lost 4 % (72 -> 75 us) and keep the odometer.
+template <typename Word, int V, int ND>
+struct SmallRuns {
+  uint32_t off[V];
+  uint32_t k1;
+  __device__ __forceinline__ SmallRuns(const BlkArgs& a, uint32_t rel) : k1(a.Q - rel) {
+#pragma unroll
+    for (int v = 0; v < V; ++v) {
+      const uint32_t c = rel + (uint32_t)v;
+      off[v] = blk_src<ND>(a, c < a.Q ? c : c - a.Q) * (uint32_t)sizeof(Word);
+    }
+  }
+  // block and source byte of the two periods of the chunk at run word w0
+  __device__ __forceinline__ void bases(const BlkArgs& a, uint32_t w0, uint32_t (&k)[2],
+                                        uint32_t (&y)[2]) const {
+    const uint32_t per = a.fnQ.d, h = a.fQ.div(w0);
+    k[0] = k[1] = a.fnQ.div(h);
+    const uint32_t o = h - k[0] * per;
+    y[0] = y[1] = blk_src<ND>(a, o * a.Q) * (uint32_t)sizeof(Word);
+    if (k1 < (uint32_t)V) {
+      k[1] += o + 1 == per;
+      y[1] = o + 1 == per ? 0 : blk_src<ND>(a, (o + 1) * a.Q) * (uint32_t)sizeof(Word);
+    }
+  }
+};
+
 // Dense layout (blocks whose size is not a multiple of 16 bytes, or a
 // tensor address that is not 16-byte aligned): the workgroup's nf blocks are
 // one run [g0, g1) (offsets from data) kept in LDS at its address modulo 16
@@ -2532,7 +2573,7 @@ __device__ __forceinline__ uint32_t blk_lds(const BlkArgs& a, uint32_t k, uint32
 // time and stored with one 16-byte store (with pattern offsets when P
 // threads divide the workgroup, else through the digit odometer); the run's
 // two edge chunks are stored word by word.
-template <typename Word, int V, int ND>
+template <typename Word, int V, int ND, bool SMALL>
 __device__ __forceinline__ void block_run(const BlkArgs& a, const uint64_t f0, const uint32_t nf,
                                           unsigned char* lds) {
   constexpr uint32_t w = sizeof(Word);
@@ -2614,6 +2655,29 @@ __device__ __forceinline__ void block_run(const BlkArgs& a, const uint64_t f0, c
     }
     return;
   }
+  if constexpr (SMALL && V >= 8) {
+    if (a.Q && nt % a.PQ == 0) {
+      const uint32_t shw = sh / w;
+      const SmallRuns<Word, V, ND> sr(a, (V * (tid % a.PQ) + a.Q - shw % a.Q) % a.Q);
+      for (uint32_t t = tid; t < n16; t += nt) {
+        const int64_t cs = a0 + 16 * (int64_t)t;
+        if (cs < g0 || cs + 16 > g1) {
+          edge(cs);
+          continue;
+        }
+        uint32_t k[2], y[2];
+        sr.bases(a, V * t - shw, k, y);
+        const uint32_t b0 = sh + k[0] * (uint32_t)a.F + y[0], b1 = sh + k[1] * (uint32_t)a.F + y[1];
+        Packed<Word, V> tmp;
+#pragma unroll
+        for (int v = 0; v < V; ++v)
+          tmp.e[v] = *reinterpret_cast<const Word*>(
+              lds + lds_off(((uint32_t)v < sr.k1 ? b0 : b1) + sr.off[v], a.pad));
+        *reinterpret_cast<typename Packed<Word, V>::P*>(a.data + cs) = tmp.p;
+      }
+      return;
+    }
+  }
   for (uint32_t t = tid; t < n16; t += nt) {
     const int64_t cs = a0 + 16 * (int64_t)t;
     if (V == 1 || cs < g0 || cs + 16 > g1) {
@@ -2682,13 +2746,13 @@ __device__ __forceinline__ void block_run(const BlkArgs& a, const uint64_t f0, c
 }
 
 // f0: first block of the workgroup's K blocks
-template <typename Word, int V, int ND>
+template <typename Word, int V, int ND, bool SMALL = false>
 __device__ __forceinline__ void block_body(const BlkArgs& a, const uint64_t f0, unsigned char* lds) {
   constexpr uint32_t w = sizeof(Word);
   const uint32_t nf = (uint32_t)((a.B - f0) < a.K ? (a.B - f0) : a.K);
   const uint32_t tid = threadIdx.x, nt = blockDim.x;
   if (a.dense) {
-    block_run<Word, V, ND>(a, f0, nf, lds);
+    block_run<Word, V, ND, SMALL>(a, f0, nf, lds);
     return;
   }
   // blocks of whole 16-byte chunks at an aligned address: the workgroup's nf
@@ -2746,7 +2810,29 @@ __device__ __forceinline__ void block_body(const BlkArgs& a, const uint64_t f0, 
       for (int v = 0; v < V; ++v) tmp.e[v] = *reinterpret_cast<const Word*>(lds + base + off[v]);
       *reinterpret_cast<typename Packed<Word, V>::P*>(out + (uint64_t)t * 16) = tmp.p;
     }
-  } else if (V > 1 && ((uint64_t)nf * a.F) % 16 == 0 && ((uintptr_t)out & 15) == 0) {
+    return;
+  }
+  if constexpr (SMALL && V >= 8) {
+    if (a.Q && nt % a.PQ == 0 && ((uint64_t)nf * a.F) % 16 == 0 && ((uintptr_t)out & 15) == 0) {
+      const uint32_t total = (uint32_t)((uint64_t)nf * a.F / 16);
+      const SmallRuns<Word, V, ND> sr(a, V * (tid % a.PQ) % a.Q);
+      for (uint32_t t = tid; t < total; t += nt) {
+        uint32_t k[2], y[2];
+        sr.bases(a, V * t, k, y);
+        const uint32_t b0 = k[0] * a.Fl, b1 = k[1] * a.Fl;
+        Packed<Word, V> tmp;
+#pragma unroll
+        for (int v = 0; v < V; ++v) {
+          const bool first = (uint32_t)v < sr.k1;
+          tmp.e[v] = *reinterpret_cast<const Word*>(
+              lds + (first ? b0 : b1) + lds_off((first ? y[0] : y[1]) + sr.off[v], a.pad));
+        }
+        *reinterpret_cast<typename Packed<Word, V>::P*>(out + (uint64_t)t * 16) = tmp.p;
+      }
+      return;
+    }
+  }
+  if (V > 1 && ((uint64_t)nf * a.F) % 16 == 0 && ((uintptr_t)out & 15) == 0) {
     // 16-byte stores: chunk t of the run is words t*V .. t*V+V-1 (cells of
     // one or several words, possibly of two blocks).  The first word's
     // block, cell and source come from divisions; each following word's from
@@ -2830,7 +2916,7 @@ __device__ __forceinline__ void block_body(const BlkArgs& a, const uint64_t f0, 
 template <typename Word, int V, int ND>
 __global__ __launch_bounds__(512) void k_block(BlkArgs a, int remap) {
   extern __shared__ __align__(16) unsigned char lds[];
-  block_body<Word, V, ND>(a, (uint64_t)xcd_logical(blockIdx.x, gridDim.x, remap) * a.K, lds);
+  block_body<Word, V, ND, true>(a, (uint64_t)xcd_logical(blockIdx.x, gridDim.x, remap) * a.K, lds);
 }
 
 const void* block_table_device(const BlockTable& t, hipError_t* err) {
@@ -2864,7 +2950,8 @@ hipError_t launch_block_w(BlkArgs a, int vec, int64_t lds, int64_t groups, const
     threads = (int)std::min<int64_t>(512, std::max<int64_t>(64, ((words + UNR - 1) / UNR + 63) / 64 * 64));
   }
   // pattern stores want a whole number of periods per workgroup's threads
-  if (vec && V > 1 && a.P) threads = std::max<int>((int)a.P, threads / (int)a.P * (int)a.P);
+  if (const int P = (int)(a.P ? a.P : a.PQ); vec && V > 1 && P)
+    threads = std::max<int>(P, threads / P * P);
   // digit tables of at most 4 digits (nearly all) run the 4-digit kernels
   const bool d4 = a.ndig <= 4;
   if (vec && V > 1 && d4)
@@ -2952,6 +3039,18 @@ hipError_t prepare_block_args(const Op& op, char* data, const LaunchCfg& cfg, Bl
   for (int k = 0; k < 8; ++k) {
     a.frad[k].init(k < t.ndig ? t.radix[k] : 1);
     a.stride[k] = k < t.ndig ? t.stride[k] : 0;
+  }
+  a.Q = a.PQ = 0;
+  if (!a.P && a.wpc == 1 && V >= 8 && t.ndig && a.frad[0].d < (uint64_t)V) {
+    int64_t Q = 1;
+    for (int k = 0; k < t.ndig && Q < V; ++k) Q *= t.radix[k];
+    const int64_t PQ = Q / gcd64(Q, V);
+    if (Q >= V && PQ <= 512) {
+      a.Q = (uint32_t)Q;
+      a.PQ = (uint32_t)PQ;
+      a.fQ.init(a.Q);
+      a.fnQ.init(a.n / a.Q);
+    }
   }
   const int64_t groups = (op.B + K - 1) / K;
   if (groups >= (1ll << 31)) return hipErrorInvalidValue;
