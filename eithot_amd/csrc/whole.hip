@@ -310,9 +310,10 @@ __device__ __forceinline__ void resident_body(const WholeGeom& g, char* data, ui
 }
 
 // One tile, or two, per workgroup.  The workgroups of a region have
-// consecutive block indices, and workgroups start in that order on each XCD, so those of the
-// earliest unfinished region all run as soon as that many are resident, which the planner keeps to half of the chip's room; they wait
-// for nobody else.  Launches of resident passes on one device follow each
+// consecutive block indices, and workgroups start in that order on each XCD,
+// so those of the earliest unfinished region all run as soon as that many are
+// resident, which the planner keeps to half of the chip's room; they wait for
+// nobody else.  Launches of resident passes on one device follow each
 // other (the runtime chains them), so no two share that room.
 template <int WL, bool MULTI, int ND, bool PAIR>
 __global__ __launch_bounds__(1024) void k_resident(WholeGeom g, char* data, WholeCtl c) {
@@ -330,7 +331,7 @@ struct WholeOp {
   char* data;
   int variant;  // log2(word) * 4 + (runs over several dims) * 2 + (at most 4 dims)
 };
-__global__ __launch_bounds__(256) void k_resident_batch(const WholeOp* __restrict__ ops,
+__global__ __launch_bounds__(kWholeBatchThreads) void k_resident_batch(const WholeOp* __restrict__ ops,
                                                         const WholeItem* __restrict__ items,
                                                         WholeCtl c) {
   extern __shared__ __align__(16) unsigned char lds[];

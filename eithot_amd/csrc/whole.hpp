@@ -239,7 +239,7 @@ WholePass plan_whole(const int64_t* dims, const int* perm1, int rank, size_t ele
 
 // The resident pass of a tensor among many in one launch: 32 KiB tiles,
 // workgroups of kWholeBatchThreads.
-constexpr int kWholeBatchThreads = 256;
+constexpr int kWholeBatchThreads = 512;
 WholePass plan_whole_batched(const int64_t* dims, const int* perm1, int rank, size_t elem, int cus,
                              int64_t lds_max);
 

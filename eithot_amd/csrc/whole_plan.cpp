@@ -262,7 +262,11 @@ WholePass plan_whole_batched(const int64_t* dims, const int* perm1, int rank, si
   if (!canonical(dims, perm1, rank, elem, c) || c.B > (int64_t)kWholeRegions) return none;
   std::vector<int> cls(c.d.size());
   for (size_t k = 0; k < cls.size(); ++k) cls[k] = (int)k;
-  constexpr int64_t kLds = 38 * 1024;  // of every workgroup of the launch
+  // of every workgroup of the launch: three of 512 threads to a CU.  512
+  // tensors of 1.5 GB took 1115 us, with two larger ones to a CU 1157, with
+  // three of 384 or 256 threads 1210 and 1396, with four 1190 (38 KiB, 256
+  // threads; 1303 of 512); 40 tensors 148 us, 192, 153 and 200, and 200
+  constexpr int64_t kLds = 52 * 1024;
   if (kLds > lds_max || !choose(c, cls, kLds, kWholeBatchThreads * kWholeHold, w.g, true)) return none;
   // large regions: two tiles per workgroup, so that fewer of them wait for
   // the rest of their region to start
