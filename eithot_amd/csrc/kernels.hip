@@ -3542,6 +3542,50 @@ __global__ __launch_bounds__(512) void k_batch_cycles(const BatchOpDev* __restri
 
 }  // namespace
 
+size_t table_bytes(const Op& op) {
+  if (op.kind == OP_CYCLE && op.cyc && !op.cyc->segs.empty())
+    return op.cyc->segs.size() * sizeof(CycleSeg) + op.cyc->slots.size() * 4;
+  if (op.kind == OP_BLOCK && op.blk && !op.blk->ndig)
+    return op.blk->src.size() * (op.blk->cells <= 65536 ? 2 : 4);
+  return 0;
+}
+
+size_t table_layout(const Plan& plan, std::vector<size_t>& offsets) {
+  size_t used = 0;
+  offsets.assign(plan.ops.size(), 0);
+  for (size_t i = 0; i < plan.ops.size(); ++i) {
+    offsets[i] = used;
+    used += (table_bytes(plan.ops[i]) + 255) / 256 * 256;
+  }
+  return used;
+}
+
+hipError_t copy_tables(const Plan& plan, char* dst, hipStream_t stream) {
+  std::vector<size_t> at;
+  std::vector<std::vector<uint16_t>> idx16;  // alive until the copies are done
+  table_layout(plan, at);
+  hipError_t e = hipSuccess;
+  for (size_t i = 0; i < plan.ops.size() && e == hipSuccess; ++i) {
+    const Op& op = plan.ops[i];
+    if (!table_bytes(op)) continue;
+    if (op.kind == OP_CYCLE) {
+      const size_t sb = op.cyc->segs.size() * sizeof(CycleSeg), lb = op.cyc->slots.size() * 4;
+      e = hipMemcpyAsync(dst + at[i], op.cyc->segs.data(), sb, hipMemcpyHostToDevice, stream);
+      if (e == hipSuccess && lb)
+        e = hipMemcpyAsync(dst + at[i] + sb, op.cyc->slots.data(), lb, hipMemcpyHostToDevice, stream);
+    } else if (op.blk->cells <= 65536) {
+      idx16.emplace_back(op.blk->src.begin(), op.blk->src.end());
+      e = hipMemcpyAsync(dst + at[i], idx16.back().data(), idx16.back().size() * 2,
+                         hipMemcpyHostToDevice, stream);
+    } else {
+      e = hipMemcpyAsync(dst + at[i], op.blk->src.data(), op.blk->src.size() * 4,
+                         hipMemcpyHostToDevice, stream);
+    }
+  }
+  const hipError_t done = hipStreamSynchronize(stream);
+  return e == hipSuccess ? done : e;
+}
+
 hipError_t prepare_op(const Op& op) {
   hipError_t e = hipSuccess;
   if (op.kind == OP_CYCLE && op.cyc && !op.cyc->segs.empty()) cycle_table_device(*op.cyc, &e);

@@ -47,6 +47,13 @@ hipError_t launch_cycle16(const Op& op, char* data, char* scratch, int64_t scrat
 // capturing the op into a graph.
 hipError_t prepare_op(const Op& op);
 
+// Pass tables in memory that the caller gives, for launch_op's `table`: the
+// bytes of an op's table (0 when it reads none), every op's offset (multiples
+// of 256) and the bytes of all, and their copy to `dst`, waited for.
+size_t table_bytes(const Op& op);
+size_t table_layout(const Plan& plan, std::vector<size_t>& offsets);
+hipError_t copy_tables(const Plan& plan, char* dst, hipStream_t stream);
+
 // While in scope, pass tables uploaded by this thread are charged to `*c`
 // (added on upload, subtracted when freed); the counter must outlive them.
 struct TableAccount {

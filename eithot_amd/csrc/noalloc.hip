@@ -26,7 +26,6 @@
 namespace {
 
 constexpr size_t kNoAllocBytes = 64ull << 20;
-constexpr size_t kAlign = 256;
 
 static __device__ __align__(256) char scratch[kNoAllocBytes];
 
@@ -50,34 +49,11 @@ eithot::LruCache<eithot::Plan>& plans() {
   return *c;
 }
 
-size_t align_up(size_t n) { return (n + kAlign - 1) / kAlign * kAlign; }
-
-// Device table bytes of one op (0 when it reads none), laid out as the
-// launcher uploads them.
-size_t table_bytes(const eithot::Op& op) {
-  if (op.kind == eithot::OP_CYCLE && op.cyc && !op.cyc->segs.empty())
-    return op.cyc->segs.size() * sizeof(eithot::CycleSeg) + op.cyc->slots.size() * 4;
-  if (op.kind == eithot::OP_BLOCK && op.blk && !op.blk->ndig)
-    return op.blk->src.size() * (op.blk->cells <= 65536 ? 2 : 4);
-  return 0;
-}
-
-// Offsets of the pass tables (each on a 256-byte boundary), and of the
-// scratch after them.
-size_t layout(const eithot::Plan& plan, std::vector<size_t>& toff) {
-  size_t used = 0;
-  toff.assign(plan.ops.size(), 0);
-  for (size_t i = 0; i < plan.ops.size(); ++i) {
-    const size_t tb = table_bytes(plan.ops[i]);
-    if (!tb) continue;
-    toff[i] = used;
-    used += align_up(tb);
-  }
-  return used;
-}
+// bytes of the array a plan uses: its tables, then its scratch
 size_t needs(const eithot::Plan& plan) {
   std::vector<size_t> toff;
-  return layout(plan, toff) + align_up((size_t)std::max<int64_t>(plan.scratch_bytes, 0));
+  return eithot::table_layout(plan, toff) +
+         ((size_t)std::max<int64_t>(plan.scratch_bytes, 0) + 255) / 256 * 256;
 }
 
 eithot::PlanPtr plan_noalloc(const eithot::Device* d, const int64_t* dims, const int* perm,
@@ -136,7 +112,7 @@ extern "C" int eithot_transpose_noalloc(void* dev, const int64_t* dims, const in
   PlanPtr plan = plan_noalloc(d, dims, perm, order, elem_bytes, n_sub, alpha, &rc);
   if (!plan) return fail(rc, "planning failed (%d)", rc);
   std::vector<size_t> toff;
-  const size_t scratch_off = layout(*plan, toff), used = needs(*plan);
+  const size_t scratch_off = table_layout(*plan, toff), used = needs(*plan);
   if (used > kNoAllocBytes)
     return fail(EITHOT_ERR_NOMEM,
                 "the plan needs %zu bytes of scratch and pass tables; the static scratch of "
@@ -148,31 +124,12 @@ extern "C" int eithot_transpose_noalloc(void* dev, const int64_t* dims, const in
   const bool fresh = st.resident.lock() != plan;
   lk.unlock();
   if (fresh) {
-    std::vector<uint16_t> idx16;
-    for (size_t i = 0; i < plan->ops.size(); ++i) {
-      const Op& op = plan->ops[i];
-      if (!table_bytes(op)) continue;
-      char* dst = base + toff[i];
-      hipError_t e = hipSuccess;
-      if (op.kind == OP_CYCLE) {
-        const size_t sb = op.cyc->segs.size() * sizeof(CycleSeg);
-        e = hipMemcpy(dst, op.cyc->segs.data(), sb, hipMemcpyHostToDevice);
-        if (e == hipSuccess && !op.cyc->slots.empty())
-          e = hipMemcpy(dst + sb, op.cyc->slots.data(), op.cyc->slots.size() * 4,
-                        hipMemcpyHostToDevice);
-      } else if (op.blk->cells <= 65536) {
-        idx16.assign(op.blk->src.begin(), op.blk->src.end());
-        e = hipMemcpy(dst, idx16.data(), idx16.size() * 2, hipMemcpyHostToDevice);
-      } else {
-        e = hipMemcpy(dst, op.blk->src.data(), op.blk->src.size() * 4, hipMemcpyHostToDevice);
-      }
-      if (e != hipSuccess) {
-        lk.lock();
-        st.resident.reset();
-        return fail(EITHOT_ERR_DEVICE, "copying pass tables failed: %s", hipGetErrorString(e));
-      }
-    }
+    const hipError_t e = copy_tables(*plan, base, stream);
     lk.lock();
+    if (e != hipSuccess) {
+      st.resident.reset();
+      return fail(EITHOT_ERR_DEVICE, "copying pass tables failed: %s", hipGetErrorString(e));
+    }
     st.resident = plan;
     lk.unlock();
   }

@@ -6,9 +6,11 @@
 #include <cstdarg>
 #include <cstdio>
 #include <cstring>
+#include <functional>
 #include <map>
 #include <memory>
 #include <mutex>
+#include <new>
 #include <sstream>
 #include <string>
 #include <vector>
@@ -195,13 +197,9 @@ void Device::trim_locked(int64_t budget, const Plan* keep) {
   }
 }
 
-bool stream_captured(hipStream_t stream);
-
 int Device::reserve_arena_locked(int64_t bytes, hipStream_t stream) {
   if (bytes <= 0) return EITHOT_OK;
-  // earlier async users of the arena must finish first (a captured call has
-  // nothing to wait for yet: its replays come later)
-  if (arena_ready && !stream_captured(stream)) {
+  if (arena_ready) {  // earlier async users of the arena must finish first
     if (hipStreamWaitEvent(stream, arena_ready, 0) != hipSuccess)
       return fail(EITHOT_ERR_DEVICE, "hipStreamWaitEvent failed");
   }
@@ -224,9 +222,6 @@ int Device::reserve_arena_locked(int64_t bytes, hipStream_t stream) {
 }
 
 int Device::release_arena_after_locked(hipStream_t stream) {
-  // an event recorded into a capture would order nothing, and could not be
-  // waited for by eager calls
-  if (stream_captured(stream)) return EITHOT_OK;
   if (!arena_ready && hipEventCreateWithFlags(&arena_ready, hipEventDisableTiming) != hipSuccess)
     return fail(EITHOT_ERR_DEVICE, "hipEventCreate failed");
   if (hipEventRecord(arena_ready, stream) != hipSuccess)
@@ -293,11 +288,6 @@ int Device::whole_end_locked(hipStream_t stream) {
 
 int Device::launch_whole_locked(const Plan& plan, char* data, hipStream_t stream) {
   const bool chain = plan.whole->mode == WHOLE_RESIDENT;
-  // a plan called once can be captured into a graph, where it runs its
-  // ordinary passes: their tables are uploaded all the same
-  if (chain && plan.table_bytes > 0 && plan.device_table_bytes(id) < plan.table_bytes)
-    for (const Op& o : plan.ops)
-      if (prepare_op(o) != hipSuccess) return fail(EITHOT_ERR_DEVICE, "uploading a pass table failed");
   int rc = chain ? whole_begin_locked(stream) : EITHOT_OK;
   if (rc) return rc;
   const hipError_t e = launch_whole(*plan.whole, data, whole_ctl, stream);
@@ -424,7 +414,8 @@ void seg_orders(const Plan& plan, int base_remap, hipStream_t stream, std::vecto
 }  // namespace
 
 int run_plan(Device* d, const Plan& plan, char* data, char* scratch, int64_t scratch_bytes,
-             hipStream_t stream, std::vector<float>* times, int64_t min_groups_cap) {
+             hipStream_t stream, std::vector<float>* times, int64_t min_groups_cap,
+             const char* tables) {
   std::vector<hipEvent_t> ev;
   if (times) {
     const std::vector<hipEvent_t>& pool = timing_events(plan.ops.size() + 1);
@@ -449,11 +440,14 @@ int run_plan(Device* d, const Plan& plan, char* data, char* scratch, int64_t scr
   std::vector<int> remap;
   std::vector<std::pair<hipEvent_t, hipEvent_t>> rec;
   if (!whole) seg_orders(plan, cfg.xcd_remap, stream, remap, rec);
+  std::vector<size_t> toff;
+  if (tables) table_layout(plan, toff);
   for (size_t i = 0; !whole && i < plan.ops.size(); ++i) {
     LaunchCfg c = cfg;
     c.xcd_remap = remap[i];
     if (rec[i].first && hipEventRecord(rec[i].first, stream) != hipSuccess) (void)hipGetLastError();
-    hipError_t e = launch_op(plan.ops[i], data, scratch, scratch_bytes, c, stream);
+    const void* table = tables && table_bytes(plan.ops[i]) ? tables + toff[i] : nullptr;
+    hipError_t e = launch_op(plan.ops[i], data, scratch, scratch_bytes, c, stream, table);
     if (e == hipSuccess && rec[i].second && hipEventRecord(rec[i].second, stream) != hipSuccess)
       (void)hipGetLastError();
     if (e != hipSuccess) {
@@ -500,6 +494,118 @@ int validate(const void* dev, const int64_t* dims, const int* perm, int order, s
   return EITHOT_OK;
 }
 
+// ---------------------------------------------------------------------------
+// captured calls
+// ---------------------------------------------------------------------------
+// A call captured into a graph runs when the graph is replayed: later than
+// any number of other calls, which grow, trim or use the arena and drop
+// tables, and beside calls on other streams.  So it uses neither: it has
+// memory of its own for its scratch and tables, which the graph owns and lets
+// go of with its last executable.
+struct GraphMem {
+  Device* d;
+  void* p;
+  GraphMem* next;
+};
+
+namespace {
+
+// Lets this thread allocate and copy while it, or another thread, captures.
+struct RelaxedCapture {
+  hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+  RelaxedCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+  ~RelaxedCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+};
+
+// Called by the HIP runtime when the last graph with the memory is gone (on
+// any of its threads; it may not call the runtime).
+void graph_mem_release(void* q) {
+  auto* m = static_cast<GraphMem*>(q);
+  m->next = m->d->retired.load(std::memory_order_relaxed);
+  while (!m->d->retired.compare_exchange_weak(m->next, m)) {
+  }
+}
+
+// Memory for the tables and scratch of `plan`, owned by the graph that
+// `stream` is captured into, with the tables in place.
+int graph_memory(Device* d, const Plan& plan, hipStream_t stream, size_t bytes, char** out) {
+  RelaxedCapture relaxed;
+  hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+  unsigned long long id = 0;
+  hipGraph_t graph = nullptr;
+  const hipGraphNode_t* deps = nullptr;
+  size_t ndeps = 0;
+  if (hipStreamGetCaptureInfo_v2(stream, &status, &id, &graph, &deps, &ndeps) != hipSuccess ||
+      status != hipStreamCaptureStatusActive || !graph)
+    return fail(EITHOT_ERR_DEVICE, "the stream's capture is not active");
+  void* p = nullptr;
+  if (hipMalloc(&p, bytes) != hipSuccess) {
+    (void)hipGetLastError();
+    return fail(EITHOT_ERR_NOMEM, "%zu bytes of scratch and tables of a captured call not available",
+                bytes);
+  }
+  hipStream_t side = nullptr;  // the null stream could not be used beside every capture
+  hipError_t e = hipStreamCreateWithFlags(&side, hipStreamNonBlocking);
+  if (e == hipSuccess) e = copy_tables(plan, (char*)p, side);
+  if (side) (void)hipStreamDestroy(side);
+  auto* m = new (std::nothrow) GraphMem{d, p, nullptr};
+  if (!m) e = hipErrorOutOfMemory;
+  hipUserObject_t obj = nullptr;
+  if (e == hipSuccess)
+    e = hipUserObjectCreate(&obj, m, graph_mem_release, 1, hipUserObjectNoDestructorSync);
+  if (e == hipSuccess) {
+    e = hipGraphRetainUserObject(graph, obj, 1, hipGraphUserObjectMove);
+    if (e != hipSuccess) {
+      (void)hipUserObjectRelease(obj, 1);  // which hands the memory back
+      m = nullptr;
+    }
+  } else {
+    (void)hipFree(p);
+    delete m;
+    m = nullptr;
+  }
+  if (!m) return fail(EITHOT_ERR_DEVICE, "memory of a captured call: %s", hipGetErrorString(e));
+  *out = (char*)p;
+  return EITHOT_OK;
+}
+
+int transpose_captured(Device* d, PlanPtr plan, const std::function<PlanPtr(int*)>& smaller, char* dev,
+                       hipStream_t stream) {
+  char* own = nullptr;
+  size_t tables = 0, bytes = 0;
+  while (!(plan->whole && plan->whole->mode == WHOLE_ORBIT)) {
+    std::vector<size_t> toff;
+    tables = table_layout(*plan, toff);
+    bytes = tables + (size_t)std::max<int64_t>(plan->scratch_bytes, 0);
+    if (!bytes) break;
+    int rc = graph_memory(d, *plan, stream, bytes, &own);
+    if (rc == EITHOT_OK) break;
+    if (rc != EITHOT_ERR_NOMEM || !plan->small_cells) return rc;
+    // small cells' tables find no place: the passes without them may
+    if (!(plan = smaller(&rc))) return rc;
+  }
+  std::lock_guard<std::mutex> lk(d->enqueue_mu);
+  std::vector<float>* times = g_timing ? &g_pass_ms : nullptr;
+  const int rc = run_plan(d, *plan, dev, plan->scratch_bytes > 0 ? own + tables : nullptr,
+                          plan->scratch_bytes, stream, times, 0, tables ? own : nullptr);
+  if (rc == EITHOT_OK) g_peak = (size_t)d->held_bytes() + (own ? bytes : 0);
+  return rc;
+}
+
+}  // namespace
+
+void Device::free_retired() {
+  GraphMem* m = retired.exchange(nullptr);
+  if (!m) return;
+  RelaxedCapture relaxed;
+  while (m) {
+    GraphMem* next = m->next;
+    (void)hipFree(m->p);  // waits for the device
+    delete m;
+    m = next;
+  }
+}
+
 static int transpose_impl(void* dev, const int64_t* dims, const int* perm, int order, size_t elem,
                           int n_sub, double alpha, hipStream_t stream, bool sync) {
   g_err.clear();
@@ -520,23 +626,12 @@ static int transpose_impl(void* dev, const int64_t* dims, const int* perm, int o
     return rc;
   }
   if ((rc = d->whole_status())) return rc;
-  // small cells' passes need tables where others need none: a captured call
-  // without an earlier one to upload them takes the others
-  if (plan->small_cells && stream_captured(stream)) {
-    bool ready;
-    {
-      std::lock_guard<std::mutex> lk(d->enqueue_mu);
-      ready = d->arena_bytes >= plan->scratch_bytes &&
-              std::all_of(plan->ops.begin(), plan->ops.end(), [&](const Op& o) {
-                return !((o.cyc && !o.cyc->segs.empty() && !o.cyc->dev.has(d->id)) ||
-                         (o.blk && !o.blk->ndig && !o.blk->dev.has(d->id)));
-              });
-    }
-    if (!ready && !(plan = d->plan_for(dims, perm, order, elem, n_sub, alpha, &rc, false))) {
-      if (!g_err.size()) fail(rc, "planning failed (%d)", rc);
-      return rc;
-    }
-  }
+  d->free_retired();
+  if (stream_captured(stream))
+    return transpose_captured(
+        d, plan,
+        [&](int* err) { return d->plan_for(dims, perm, order, elem, n_sub, alpha, err, false); },
+        (char*)dev, stream);
   {
     std::lock_guard<std::mutex> lk(d->enqueue_mu);
     const bool whole = d->takes_whole_locked(*plan, stream);
@@ -544,15 +639,12 @@ static int transpose_impl(void* dev, const int64_t* dims, const int* perm, int o
     // plan's own need when one footprint exceeds it, or the holding floor
     // (which spares calls on small tensors from evicting and re-uploading
     // the tables of the others)
-    // a resident pass needs no extra memory, but keeps what a captured call of
-    // its plan will use
-    const bool keeps = !whole || plan->whole->mode == WHOLE_RESIDENT;
-    const int64_t own = keeps ? plan->scratch_bytes + plan->table_bytes : 0;
+    const int64_t own = whole ? 0 : plan->scratch_bytes + plan->table_bytes;
     const int64_t budget = std::max<int64_t>(
         std::max<int64_t>((int64_t)(alpha * (double)plan->tensor_bytes), own),
         tuning_get().hold_floor);
-    d->trim_locked(budget, keeps ? plan.get() : nullptr);
-    if (whole ? keeps && d->arena_bytes < plan->scratch_bytes : plan->scratch_bytes > 0) {
+    d->trim_locked(budget, whole ? nullptr : plan.get());
+    if (!whole && plan->scratch_bytes > 0) {
       rc = d->reserve_arena_locked(plan->scratch_bytes, stream);
       if (rc) return rc;
     }
@@ -617,6 +709,7 @@ void eithot_release(void) {
   if (!d) return;
   std::vector<PlanPtr> dropped;
   std::lock_guard<std::mutex> lk(d->enqueue_mu);
+  d->free_retired();
   (void)hipDeviceSynchronize();
   if (d->arena) (void)hipFree(d->arena);
   d->arena = nullptr;

@@ -25,6 +25,8 @@ using PlanPtr = std::shared_ptr<const Plan>;
 //              shrinking, table eviction and every launch that uses them are
 //              mutually exclusive, so no thread launches into memory another
 //              thread frees.  Lock order: enqueue_mu, then mu.
+struct GraphMem;
+
 struct Device {
   int id = 0;
   DeviceProfile prof;
@@ -69,6 +71,11 @@ struct Device {
   // user on `stream`.
   int reserve_arena_locked(int64_t bytes, hipStream_t stream);
   int release_arena_after_locked(hipStream_t stream);
+  // Memory that graphs have let go of (GraphMem, chained), freed by the next
+  // call.  Not under enqueue_mu: graphs end on any thread.
+  std::atomic<GraphMem*> retired{nullptr};
+  void free_retired();
+
   // With enqueue_mu held: whether a call of `plan` on `stream` runs its
   // whole-permutation pass, and the launch of it.  Resident passes are left
   // out of stream captures (a replay could not be chained).
@@ -95,8 +102,10 @@ void set_peak(size_t bytes);
 int validate(const void* dev, const int64_t* dims, const int* perm, int order, size_t elem);
 // Enqueues the plan's passes on `stream`.  min_groups_cap > 0 lowers the
 // launch configuration's workgroup floor per pass to at most that (callers
-// whose passes share the GPU with other work).
+// whose passes share the GPU with other work).  tables: the passes' tables as
+// copy_tables lays them out, instead of the plan's own copies.
 int run_plan(Device* d, const Plan& plan, char* data, char* scratch, int64_t scratch_bytes,
-             hipStream_t stream, std::vector<float>* times, int64_t min_groups_cap = 0);
+             hipStream_t stream, std::vector<float>* times, int64_t min_groups_cap = 0,
+             const char* tables = nullptr);
 
 }  // namespace eithot

@@ -57,7 +57,12 @@ int eithot_transpose(void* dev, const int64_t* dims, const int* perm, int order,
  * arena stays reserved until the work completes; do not free `dev` first.
  * Calls may come from several threads: the launches of calls that use the
  * arena or pass tables are enqueued one call at a time, and a call's first
- * pass waits (on the device) for the last pass of the previous arena user. */
+ * pass waits (on the device) for the last pass of the previous arena user.
+ * On a stream under capture the call's scratch and tables are memory of its
+ * own (within the same bound, counted by eithot_last_peak_extra_bytes of the
+ * capturing call), which the graph owns: replays may come at any time and
+ * beside any other call.  The memory is freed by the first transpose or
+ * eithot_release after the graph and its executables are destroyed. */
 int eithot_transpose_async(void* dev, const int64_t* dims, const int* perm, int order,
                            size_t elem_bytes, int n_sub, double alpha, void* stream);
 
