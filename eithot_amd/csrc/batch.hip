@@ -58,6 +58,7 @@ struct eithot_batch {
   std::vector<Plan> fwd, inv;  // a tensor that the resident launch takes keeps no passes
   std::vector<WholePass> fwd_whole, inv_whole;
   WholeBatch* whole = nullptr;  // the resident launch, before the stages
+  uint64_t whole_region = 0;    // bytes of its largest region
   std::vector<LaunchStage> stages;
   char* scratch = nullptr;
   int64_t scratch_bytes = 0;
@@ -105,6 +106,14 @@ struct eithot_batch {
     if (!prof.whole || plan.ops.size() < 2) return;
     w = plan_whole_batched(dims.data(), perm.data(), (int)dims.size(), r.elem, prof.cus, prof.lds_max);
     if (w.mode == WHOLE_NONE) return;
+    {
+      std::lock_guard<std::mutex> lk(dev->enqueue_mu);
+      if (!dev->whole_room_locked(w.g.region)) {
+        w = WholePass();
+        return;
+      }
+    }
+    whole_region = std::max(whole_region, w.g.region);
     plan.ops.clear();
     plan.scratch_bytes = 0;
   }
@@ -117,7 +126,12 @@ struct eithot_batch {
     std::stable_sort(p.begin(), p.end(), [](const auto& x, const auto& y) {
       return x.first->g.tiles > y.first->g.tiles;
     });
-    if (whole_batch_build(p, dev->whole_ctl, out) != hipSuccess)
+    WholeCtl ctl;
+    {
+      std::lock_guard<std::mutex> lk(dev->enqueue_mu);
+      ctl = dev->whole_ctl;
+    }
+    if (whole_batch_build(p, ctl, out) != hipSuccess)
       return fail(EITHOT_ERR_NOMEM, "building the batch's resident pass failed");
     return EITHOT_OK;
   }
@@ -175,10 +189,6 @@ int eithot_batch_build(eithot_batch* b, double alpha, int tune) {
   DeviceProfile prof = b->dev->profile();
   prof.cycle_shift = 0;  // batched cycle items move narrow cells word by word
   b->cfg = b->dev->launch_cfg();
-  {
-    std::lock_guard<std::mutex> lk(b->dev->enqueue_mu);
-    if (prof.whole && !b->dev->whole_init_locked()) prof.whole = 0;
-  }
   b->fwd.resize(n);
   b->inv.resize(n);
   b->fwd_whole.resize(n);
@@ -251,13 +261,14 @@ int eithot_batch_build(eithot_batch* b, double alpha, int tune) {
       if (!rc) {
         {
           std::lock_guard<std::mutex> lk(b->dev->enqueue_mu);
-          if (b->whole || whole_inv) rc = b->dev->whole_begin_locked(b->stream);
+          const bool chained = (b->whole || whole_inv) &&
+                               b->dev->whole_begin_locked(b->whole_region, b->stream);
           (void)hipEventRecord(e0, b->stream);
           if (!rc) rc = b->enqueue(b->whole, f, cfg, b->stream);
           (void)hipEventRecord(e1, b->stream);
           if (!rc) rc = b->enqueue(whole_inv, v, cfg, b->stream);
           (void)hipEventRecord(e2, b->stream);
-          if (!rc && (b->whole || whole_inv)) rc = b->dev->whole_end_locked(b->stream);
+          if (chained) b->dev->whole_end_locked(b->stream);
         }
         if (hipStreamSynchronize(b->stream) != hipSuccess) rc = EITHOT_ERR_DEVICE;
       }
@@ -268,7 +279,6 @@ int eithot_batch_build(eithot_batch* b, double alpha, int tune) {
       }
       free_stages(f);
       free_stages(v);
-      if (!rc) rc = b->dev->whole_status();
       if (rc) {
         (void)hipEventDestroy(e0);
         (void)hipEventDestroy(e1);
@@ -310,22 +320,20 @@ int eithot_batch_build(eithot_batch* b, double alpha, int tune) {
 int eithot_batch_run(eithot_batch* b, void* stream, int sync) {
   if (!b || !b->built) return fail(EITHOT_ERR_INVALID, "batch not built");
   hipStream_t s = stream ? (hipStream_t)stream : b->stream;
-  int rc = EITHOT_OK;
   if (b->whole) {
-    if ((rc = b->dev->whole_status())) return rc;
     std::lock_guard<std::mutex> lk(b->dev->enqueue_mu);
-    if (b->dev->whole_off)
-      return fail(EITHOT_ERR_DEVICE, "resident passes are off on this device: build the batch again");
-    if ((rc = b->dev->whole_begin_locked(s))) return rc;
-    if (hipGraphLaunch(b->exec, s) != hipSuccess)
-      return fail(EITHOT_ERR_DEVICE, "graph launch failed");
-    if ((rc = b->dev->whole_end_locked(s))) return rc;
+    // behind other resident passes; its words are its own, so where that is
+    // not possible it may run beside them, if slowly
+    const bool chained = b->dev->whole_begin_locked(b->whole_region, s);
+    const hipError_t e = hipGraphLaunch(b->exec, s);
+    if (chained) b->dev->whole_end_locked(s);
+    if (e != hipSuccess) return fail(EITHOT_ERR_DEVICE, "graph launch failed");
   } else if (hipGraphLaunch(b->exec, s) != hipSuccess) {
     return fail(EITHOT_ERR_DEVICE, "graph launch failed");
   }
   if (sync && hipStreamSynchronize(s) != hipSuccess)
     return fail(EITHOT_ERR_DEVICE, "batch execution failed");
-  return sync && b->whole ? b->dev->whole_status() : EITHOT_OK;
+  return EITHOT_OK;
 }
 
 int eithot_batch_info(const eithot_batch* b, int* launches, int64_t* scratch_bytes,

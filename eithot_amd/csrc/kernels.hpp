@@ -98,16 +98,14 @@ void batch_launch_free(BatchLaunch* L);
 int64_t batch_launch_items(const BatchLaunch* L);
 int batch_launch_count(const BatchLaunch* L);  // kernel launches per enqueue
 
-// The whole-permutation pass `p` over the tensor at `data` (whole.hip).  A
-// resident pass whose workgroups do not meet within ctl.patience sets
-// *ctl.host_failed and leaves the tensor indeterminate.
+// The whole-permutation pass `p` over the tensor at `data` (whole.hip).
 struct WholePass;
 struct WholeCtl;
 hipError_t launch_whole(const WholePass& p, char* data, const WholeCtl& ctl, hipStream_t stream);
 // the current device's words for single tensors (fills ctl's pointers to them)
 hipError_t whole_ctl_device(WholeCtl& ctl);
 // Resident passes (plan_whole_batched) of many tensors in one launch, with
-// words of their own; ctl gives the failure words and the patience.
+// words of their own; ctl gives the rest.
 struct WholeBatch;
 hipError_t whole_batch_build(const std::vector<std::pair<const WholePass*, char*>>& passes,
                              const WholeCtl& ctl, WholeBatch** out);

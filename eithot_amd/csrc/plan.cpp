@@ -1075,6 +1075,7 @@ static int64_t* tuning_field(Tuning& t, const char* key) {
   if (!strcmp(key, "cycle_u_depth")) return &t.cycle_u_depth;
   if (!strcmp(key, "min_groups")) return &t.min_groups;
   if (!strcmp(key, "whole")) return &t.whole;
+  if (!strcmp(key, "whole_patience")) return &t.whole_patience;
   return nullptr;
 }
 
@@ -1102,6 +1103,7 @@ int tuning_set(const char* key, int64_t value) {
   if (f == &t.lower_mask && (value == 0 || value > LOWER_ALL)) return EITHOT_ERR_INVALID;
   if (f == &t.cycle_u_depth && value != 4 && value != 6 && value != 8) return EITHOT_ERR_INVALID;
   if (f == &t.min_groups && (value < 1 || value > (1 << 20))) return EITHOT_ERR_INVALID;
+  if (f == &t.whole_patience && value > 60000000) return EITHOT_ERR_INVALID;
   const bool flag = f == &t.regroup || f == &t.lds_threads_auto || f == &t.cycle_cell_pref ||
                     f == &t.cycle_word_cost || f == &t.block_digits || f == &t.block_pad ||
                     f == &t.xcd_remap || f == &t.whole;

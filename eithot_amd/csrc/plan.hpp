@@ -269,6 +269,10 @@ struct Tuning {
   int64_t cycle_u_depth = 4;        // accepted (4, 6, 8), no effect
   int64_t min_groups = 1024;        // workgroups a single-launch pass spreads its footprints over
   int64_t whole = 1;                // whole-permutation passes (whole.hpp) where they fit
+  // microseconds that a resident pass's workgroups wait for each other: they
+  // meet within microseconds, unless other work holds the chip (ms); what
+  // follows then takes milliseconds too
+  int64_t whole_patience = 100000;
   bool plain = true;   // every knob of the passes has its default value
   uint64_t epoch = 0;  // bumped on every change (plan caches key on it)
 };

@@ -229,10 +229,6 @@ int Device::release_arena_after_locked(hipStream_t stream) {
   return EITHOT_OK;
 }
 
-// ticks of the 100 MHz clock that a resident pass waits for its workgroups
-// (20 s; they meet within microseconds unless other processes hold the chip)
-constexpr uint64_t kWholePatience = 2000000000ull;
-
 bool stream_captured(hipStream_t stream) {
   if (!stream) return false;  // the null stream cannot be
   hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
@@ -246,64 +242,53 @@ bool stream_captured(hipStream_t stream) {
 bool Device::takes_whole_locked(const Plan& plan, hipStream_t stream) {
   if (!plan.whole) return false;
   if (plan.whole->mode == WHOLE_ORBIT) return true;
-  return !whole_off && !stream_captured(stream) && whole_init_locked();
+  return !stream_captured(stream) && whole_begin_locked(plan.whole->g.region, stream);
 }
 
-bool Device::whole_init_locked() {
-  if (whole_ready) return !whole_off;
-  WholeCtl c;
-  c.patience = kWholePatience;
-  hipEvent_t ev = nullptr;
-  if (whole_off || whole_ctl_device(c) != hipSuccess ||
-      hipHostMalloc((void**)&c.host_failed, sizeof(uint32_t), hipHostMallocDefault) != hipSuccess ||
-      hipEventCreateWithFlags(&ev, hipEventDisableTiming) != hipSuccess) {
+bool Device::whole_room_locked(uint64_t region) {
+  if (!whole_ready) {
+    if (whole_ctl_device(whole_ctl) != hipSuccess ||
+        hipEventCreateWithFlags(&whole_ready, hipEventDisableTiming) != hipSuccess) {
+      (void)hipGetLastError();
+      whole_ready = nullptr;
+      return false;
+    }
+  }
+  whole_ctl.patience = (uint64_t)tuning_get().whole_patience * 100;
+  if (region <= whole_room) return true;
+  uint64_t bytes = 1ull << 20;
+  while (bytes < region) bytes *= 2;
+  char* p = nullptr;
+  if (hipHostMalloc((void**)&p, bytes, hipHostMallocDefault) != hipSuccess) {
     (void)hipGetLastError();
-    whole_off = true;
     return false;
   }
-  *c.host_failed = 0;
-  whole_ctl = c;
-  whole_ready = ev;
+  whole_ctl.room = p;
+  whole_room = bytes;
   return true;
 }
 
 // Passes on the null stream follow each other by themselves; the event is
 // recorded behind them only when a call on another stream needs it (the null
 // stream outlives every call, other streams may not).
-int Device::whole_begin_locked(hipStream_t stream) {
-  if (!stream && !whole_elsewhere) return EITHOT_OK;
-  if (!whole_elsewhere && hipEventRecord(whole_ready, nullptr) != hipSuccess)
-    return fail(EITHOT_ERR_DEVICE, "hipEventRecord failed");
-  if (hipStreamWaitEvent(stream, whole_ready, 0) != hipSuccess)
-    return fail(EITHOT_ERR_DEVICE, "hipStreamWaitEvent failed");
-  return EITHOT_OK;
+bool Device::whole_begin_locked(uint64_t region, hipStream_t stream) {
+  if (!whole_room_locked(region)) return false;
+  if (!stream && !whole_elsewhere) return true;
+  if ((!whole_elsewhere && hipEventRecord(whole_ready, nullptr) != hipSuccess) ||
+      hipStreamWaitEvent(stream, whole_ready, 0) != hipSuccess) {
+    (void)hipGetLastError();  // beside a capture, for one
+    return false;
+  }
+  return true;
 }
 
-int Device::whole_end_locked(hipStream_t stream) {
+void Device::whole_end_locked(hipStream_t stream) {
   whole_elsewhere = stream != nullptr;
-  if (stream && hipEventRecord(whole_ready, stream) != hipSuccess)
-    return fail(EITHOT_ERR_DEVICE, "hipEventRecord failed");
-  return EITHOT_OK;
-}
-
-int Device::launch_whole_locked(const Plan& plan, char* data, hipStream_t stream) {
-  const bool chain = plan.whole->mode == WHOLE_RESIDENT;
-  int rc = chain ? whole_begin_locked(stream) : EITHOT_OK;
-  if (rc) return rc;
-  const hipError_t e = launch_whole(*plan.whole, data, whole_ctl, stream);
-  if (e != hipSuccess)
-    return fail(EITHOT_ERR_DEVICE, "whole pass launch failed: %s", hipGetErrorString(e));
-  return chain ? whole_end_locked(stream) : EITHOT_OK;
-}
-
-int Device::whole_status() {
-  std::lock_guard<std::mutex> lk(enqueue_mu);
-  if (whole_off || !whole_ctl.host_failed || !*(volatile uint32_t*)whole_ctl.host_failed)
-    return EITHOT_OK;
-  whole_off = true;
-  return fail(EITHOT_ERR_DEVICE,
-              "a resident pass gave up waiting for its workgroups; the tensors of calls since the "
-              "last synchronisation are indeterminate");
+  if (stream && hipEventRecord(whole_ready, stream) != hipSuccess) {
+    (void)hipGetLastError();
+    (void)hipStreamSynchronize(stream);  // nothing is left to wait for
+    whole_elsewhere = false;
+  }
 }
 
 // Timing events of this thread on each device, reused from call to call
@@ -414,7 +399,7 @@ void seg_orders(const Plan& plan, int base_remap, hipStream_t stream, std::vecto
 }  // namespace
 
 int run_plan(Device* d, const Plan& plan, char* data, char* scratch, int64_t scratch_bytes,
-             hipStream_t stream, std::vector<float>* times, int64_t min_groups_cap,
+             hipStream_t stream, std::vector<float>* times, bool whole, int64_t min_groups_cap,
              const char* tables) {
   std::vector<hipEvent_t> ev;
   if (times) {
@@ -427,10 +412,12 @@ int run_plan(Device* d, const Plan& plan, char* data, char* scratch, int64_t scr
     }
   }
   int rc = EITHOT_OK;
-  const bool whole = d->takes_whole_locked(plan, stream);
   const size_t npass = whole ? 1 : plan.ops.size();
   if (whole) {
-    rc = d->launch_whole_locked(plan, data, stream);
+    const hipError_t e = launch_whole(*plan.whole, data, d->whole_ctl, stream);
+    if (e != hipSuccess)
+      rc = fail(EITHOT_ERR_DEVICE, "whole pass launch failed: %s", hipGetErrorString(e));
+    if (plan.whole->mode == WHOLE_RESIDENT) d->whole_end_locked(stream);
     if (rc == EITHOT_OK && times && hipEventRecord(ev[1], stream) != hipSuccess)
       rc = fail(EITHOT_ERR_DEVICE, "pass timing event failed");
     if (times) ev.resize(2);
@@ -587,7 +574,8 @@ int transpose_captured(Device* d, PlanPtr plan, const std::function<PlanPtr(int*
   std::lock_guard<std::mutex> lk(d->enqueue_mu);
   std::vector<float>* times = g_timing ? &g_pass_ms : nullptr;
   const int rc = run_plan(d, *plan, dev, plan->scratch_bytes > 0 ? own + tables : nullptr,
-                          plan->scratch_bytes, stream, times, 0, tables ? own : nullptr);
+                          plan->scratch_bytes, stream, times,
+                          d->takes_whole_locked(*plan, stream), 0, tables ? own : nullptr);
   if (rc == EITHOT_OK) g_peak = (size_t)d->held_bytes() + (own ? bytes : 0);
   return rc;
 }
@@ -625,7 +613,6 @@ static int transpose_impl(void* dev, const int64_t* dims, const int* perm, int o
     if (!g_err.size()) fail(rc, "planning failed (%d)", rc);
     return rc;
   }
-  if ((rc = d->whole_status())) return rc;
   d->free_retired();
   if (stream_captured(stream))
     return transpose_captured(
@@ -650,7 +637,7 @@ static int transpose_impl(void* dev, const int64_t* dims, const int* perm, int o
     }
     std::vector<float>* times = g_timing ? &g_pass_ms : nullptr;
     TableAccount acct(&d->cached_tables);
-    rc = run_plan(d, *plan, (char*)dev, d->arena, plan->scratch_bytes, stream, times);
+    rc = run_plan(d, *plan, (char*)dev, d->arena, plan->scratch_bytes, stream, times, whole);
     if (rc) return rc;
     if (!whole && plan->scratch_bytes > 0) {
       rc = d->release_arena_after_locked(stream);
@@ -662,7 +649,6 @@ static int transpose_impl(void* dev, const int64_t* dims, const int* perm, int o
     hipError_t e = hipStreamSynchronize(stream);
     if (e == hipSuccess) e = hipGetLastError();
     if (e != hipSuccess) return fail(EITHOT_ERR_DEVICE, "device error: %s", hipGetErrorString(e));
-    if ((rc = d->whole_status())) return rc;
   }
   return EITHOT_OK;
 }

@@ -38,13 +38,14 @@ struct Device {
   int64_t arena_bytes = 0;
   hipEvent_t arena_ready = nullptr;  // recorded after the last pass that used the arena
   // Resident whole-permutation passes share the chip with no other of their
-  // kind (whole.hip): each waits, on the device, for the one before.  Once
-  // one has given up waiting (*whole_ctl.host_failed, written by the kernel) the
-  // device runs ordinary passes only.  All under enqueue_mu.
+  // kind (whole.hip): each waits, on the device, for the one before.  All
+  // under enqueue_mu.
   hipEvent_t whole_ready = nullptr;
   bool whole_elsewhere = false;      // the last one ran on a stream other than the null stream
-  bool whole_off = false;
   WholeCtl whole_ctl;
+  // bytes at whole_ctl.room: a power of two, 1 to 64 MiB.  A smaller room
+  // before it stays, for the passes in flight and the batches that name it.
+  uint64_t whole_room = 0;
   // device bytes of the pass tables uploaded for plans of this cache (and
   // not yet freed; an evicted plan a request still holds counts until freed)
   std::atomic<int64_t> cached_tables{0};
@@ -77,18 +78,15 @@ struct Device {
   void free_retired();
 
   // With enqueue_mu held: whether a call of `plan` on `stream` runs its
-  // whole-permutation pass, and the launch of it.  Resident passes are left
-  // out of stream captures (a replay could not be chained).
+  // whole-permutation pass, which run_plan then launches.  Resident passes
+  // are left out of stream captures (a replay could not be chained).
   bool takes_whole_locked(const Plan& plan, hipStream_t stream);
-  // Resident passes on `stream` go between these two; whole_init_locked
-  // comes before the first (false: the device runs none).
-  bool whole_init_locked();
-  int whole_begin_locked(hipStream_t stream);
-  int whole_end_locked(hipStream_t stream);
-  int launch_whole_locked(const Plan& plan, char* data, hipStream_t stream);
-  // Reports (once) that a resident pass gave up: its tensor's contents are
-  // indeterminate.  EITHOT_OK otherwise.
-  int whole_status();
+  // Resident passes over regions of up to `region` bytes on `stream` go
+  // between these two (false: the device or the stream can run none now);
+  // batches, which launch later, make sure of their room.
+  bool whole_room_locked(uint64_t region);
+  bool whole_begin_locked(uint64_t region, hipStream_t stream);
+  void whole_end_locked(hipStream_t stream);
   // Device bytes the library holds for plain transposes on this device.
   int64_t held_bytes();
 };
@@ -103,9 +101,10 @@ int validate(const void* dev, const int64_t* dims, const int* perm, int order, s
 // Enqueues the plan's passes on `stream`.  min_groups_cap > 0 lowers the
 // launch configuration's workgroup floor per pass to at most that (callers
 // whose passes share the GPU with other work).  tables: the passes' tables as
-// copy_tables lays them out, instead of the plan's own copies.
+// copy_tables lays them out, instead of the plan's own copies.  whole: what
+// takes_whole_locked has said.
 int run_plan(Device* d, const Plan& plan, char* data, char* scratch, int64_t scratch_bytes,
-             hipStream_t stream, std::vector<float>* times, int64_t min_groups_cap = 0,
+             hipStream_t stream, std::vector<float>* times, bool whole, int64_t min_groups_cap = 0,
              const char* tables = nullptr);
 
 }  // namespace eithot

@@ -117,7 +117,7 @@ struct eithot_server {
         continue;
       }
       r->latency_ms = ns / 1e6;
-      r->status = r->plan->whole && dev->whole_status() ? EITHOT_ERR_DEVICE : 2;
+      r->status = 2;
       pool.release(r->off, r->bytes);
       --stream_load[r->stream];
       free_events.push_back(r->done_ev);
@@ -168,7 +168,7 @@ struct eithot_server {
         // 128 workgroups' floor per pass (2 % more tensors/s at saturation
         // than the single-launch 1024)
         rc = run_plan(dev, *r->plan, r->dev, need > 0 ? pool_mem + off : nullptr, need, st,
-                      nullptr, kServedMinGroups);
+                      nullptr, dev->takes_whole_locked(*r->plan, st), kServedMinGroups);
       }
       if (rc == EITHOT_OK && hipEventRecord(r->done_ev, st) != hipSuccess) rc = EITHOT_ERR_DEVICE;
       if (rc == EITHOT_OK && hipLaunchHostFunc(st, on_done, r) != hipSuccess) rc = EITHOT_ERR_DEVICE;

@@ -208,46 +208,84 @@ __device__ __forceinline__ void tile_store(const WholeGeom& g, const WholeTile& 
 // ---------------------------------------------------------------------------
 // resident form
 // ---------------------------------------------------------------------------
-// Counts workgroup t of the n of a region; true for the last one.  A region
-// has 16 counters (each on a line of its own: one address takes about 30 ns
-// per addition) and a root that the last workgroup of each adds to, all zero
-// between passes.
-__device__ __forceinline__ uint32_t ctl_add(uint32_t* p, uint32_t v) {
-  return __hip_atomic_fetch_add(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+struct Words {
+  static __device__ __forceinline__ uint32_t add(uint32_t* p, uint32_t v) {
+    return __hip_atomic_fetch_add(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+  static __device__ __forceinline__ uint32_t get(uint32_t* p) {
+    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+  static __device__ __forceinline__ void set(uint32_t* p, uint32_t v) {
+    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+  static __device__ __forceinline__ bool cas(uint32_t* p, uint32_t from, uint32_t to) {
+    return __hip_atomic_compare_exchange_strong(p, &from, to, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
+                                                __HIP_MEMORY_SCOPE_AGENT);
+  }
+  static __device__ __forceinline__ uint64_t now() { return __builtin_amdgcn_s_memrealtime(); }
+  static __device__ __forceinline__ void pause() { __builtin_amdgcn_s_sleep(1); }
+};
+
+// Constant memory read late: the compiler may not load through the result
+// ahead of this point.
+template <typename T>
+using Const = const T __attribute__((address_space(4)));
+template <typename T>
+__device__ __forceinline__ Const<T>* late(Const<T>* p) {
+  asm volatile("" : "+s"(p));
+  return p;
 }
-__device__ __forceinline__ uint32_t ctl_get(uint32_t* p) {
-  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-__device__ __forceinline__ void ctl_set(uint32_t* p, uint32_t v) {
-  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-__device__ __forceinline__ bool ctl_arrive(const WholeCtl& c, uint32_t slot, uint32_t t, uint32_t n) {
-  const uint32_t subs = n <= kWholeSubs ? 1 : kWholeSubs;
-  const uint32_t j = t % subs, members = (n - j + subs - 1) / subs;
-  uint32_t* sub = c.sub + (uint64_t)j * c.slots + slot;
-  if (ctl_add(sub, 1) != members - 1) return false;
-  ctl_set(sub, 0);
-  if (subs == 1) return true;
-  if (ctl_add(c.root + slot, 1) != subs - 1) return false;
-  ctl_set(c.root + slot, 0);
-  return true;
+
+// The region at `base` moved by one workgroup, in output order into host
+// memory and back: what the last workgroup does where the others have left.
+// Regions of other launches may want the host memory too; whoever holds its
+// lock runs and lets go of it.  g and c are read late: loaded with the rest
+// at the kernel's start, they and what is made of them cost every workgroup
+// registers (64 MiB of pairs: 33.6 us, 32.1 so).
+template <int WL>
+__device__ __forceinline__ void move_alone(Const<WholeGeom>* g, Const<WholeCtl>* c, char* base) {
+  using E = typename ElemOf<WL>::T;
+  uint32_t* lock = c->lock;
+  char* room = c->room;
+  uint32_t od[kWholeDims], ogin[kWholeDims];
+#pragma unroll
+  for (int k = 0; k < kWholeDims; ++k) {
+    od[k] = g->od[k];
+    ogin[k] = g->ogin[k];
+  }
+  if (threadIdx.x == 0)
+    while (!Words::cas(lock, 0, 1)) Words::pause();
+  __syncthreads();
+  __threadfence_system();
+  const uint32_t bytes = (uint32_t)g->region, n = bytes >> WL, n16 = bytes / 16;
+  for (uint32_t o = threadIdx.x; o < n; o += blockDim.x)
+    reinterpret_cast<E*>(room)[o] =
+        reinterpret_cast<const Loose<WL>*>(base + whole_source(g->r, od, ogin, o))->v;
+  __threadfence_system();  // written through, and no stale copy is read
+  __syncthreads();
+  __threadfence_system();
+  for (uint32_t o = threadIdx.x; o < n16; o += blockDim.x)
+    reinterpret_cast<V16u*>(base)[o] = reinterpret_cast<const V16*>(room)[o];
+  for (uint32_t o = n16 * 16 + threadIdx.x; o < bytes; o += blockDim.x) base[o] = room[o];
+  __threadfence_system();
+  __syncthreads();
+  if (threadIdx.x == 0) Words::set(lock, 0);
 }
 
 // Tiles t * per .. of region b, meeting its region's other workgroups at
 // `slot`.  The first is held in LDS, a second one in registers until the
 // first is stored.  No data passes between workgroups: the counters only
 // order a region's loads, which are complete once in LDS or waited for,
-// before its stores, so they need no cache flush.  The wait is bounded: after
-// `patience` ticks of the 100 MHz clock a workgroup reports a failure and
-// leaves without storing, and so do those after it.
+// before its stores, so they need no cache flush.  True when the workgroup is
+// to move the region alone, and then to set the region's word to the second
+// word of LDS.
 template <int WL, bool MULTI, int ND, bool PAIR>
-__device__ __forceinline__ void resident_body(const WholeGeom& g, char* data, uint32_t b, uint32_t t,
+__device__ __forceinline__ bool resident_body(const WholeGeom& g, char* data, uint32_t b, uint32_t t,
                                               uint32_t slot, const WholeCtl& c,
                                               unsigned char* lds) {
   uint32_t* ctl = reinterpret_cast<uint32_t*>(lds);
-  // the region is complete when this word changes
-  uint32_t closed = 0;
-  if (threadIdx.x == 0) closed = ctl_get(c.open + slot);
+  uint32_t word = 0;
+  if (threadIdx.x == 0) word = Words::get(c.open + slot);
   const WholeTile x = whole_tile<ND>(g, whole_nth(g, PAIR ? t * g.per : t));
   const uint64_t region = (uint64_t)b * g.region, room = g.B * g.region - region;
   char* base = data + region;
@@ -278,27 +316,11 @@ __device__ __forceinline__ void resident_body(const WholeGeom& g, char* data, ui
   }
   __syncthreads();
   if (threadIdx.x == 0) {
-    uint32_t ok = 1;
-    if (ctl_arrive(c, slot, t, g.wgs)) {
-      ctl_set(c.open + slot, closed + 1);
-    } else {
-      const uint64_t t0 = __builtin_amdgcn_s_memrealtime();
-      for (;;) {
-        const uint32_t failed = ctl_get(c.failed), now = ctl_get(c.open + slot);
-        if (!failed && now != closed) break;
-        if (failed || __builtin_amdgcn_s_memrealtime() - t0 > c.patience) {
-          ctl_set(c.failed, 1);
-          __hip_atomic_store(c.host_failed, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-          ok = 0;
-          break;
-        }
-        __builtin_amdgcn_s_sleep(1);
-      }
-    }
-    ctl[0] = ok;
+    ctl[0] = whole_meet<Words>(c, slot, t, g.wgs, word);
+    ctl[1] = word;
   }
   __syncthreads();
-  if (!ctl[0]) return;
+  if (ctl[0] != MEET_STORE) return ctl[0] == MEET_ALONE;
   tile_store<WL, MULTI, ND>(g, x, base + x.out, a);
   if (second) {
     __syncthreads();  // x has been read out of LDS, and its lists
@@ -307,22 +329,9 @@ __device__ __forceinline__ void resident_body(const WholeGeom& g, char* data, ui
     __syncthreads();
     tile_store<WL, MULTI, ND>(g, y, base + y.out, a);
   }
+  return false;
 }
 
-// One tile, or two, per workgroup.  The workgroups of a region have
-// consecutive block indices, and workgroups start in that order on each XCD,
-// so those of the earliest unfinished region all run as soon as that many are
-// resident, which the planner keeps to half of the chip's room; they wait for
-// nobody else.  Launches of resident passes on one device follow each
-// other (the runtime chains them), so no two share that room.
-template <int WL, bool MULTI, int ND, bool PAIR>
-__global__ __launch_bounds__(1024) void k_resident(WholeGeom g, char* data, WholeCtl c) {
-  extern __shared__ __align__(16) unsigned char lds[];
-  const uint32_t b = g.fwgs.div(blockIdx.x);
-  resident_body<WL, MULTI, ND, PAIR>(g, data, b, blockIdx.x - b * g.wgs, b, c, lds);
-}
-
-// The same over the regions of many tensors: workgroup i takes item i.
 struct WholeItem {
   uint32_t op, b, t, slot;
 };
@@ -331,6 +340,43 @@ struct WholeOp {
   char* data;
   int variant;  // log2(word) * 4 + (runs over several dims) * 2 + (at most 4 dims)
 };
+// The rest of a workgroup that resident_body has told to move region b alone.
+template <int WL>
+__device__ __forceinline__ void finish_alone(Const<WholeGeom>* g, Const<WholeCtl>* c, char* data,
+                                             uint32_t b, uint32_t slot, const unsigned char* lds) {
+  move_alone<WL>(g, c, data + (uint64_t)b * g->region);
+  if (threadIdx.x == 0)
+    whole_done_alone<Words>(c->open + slot, reinterpret_cast<const uint32_t*>(lds)[1]);
+}
+struct ResidentArgs {  // of k_resident, as it gets them
+  WholeGeom g;
+  char* data;
+  WholeCtl c;
+};
+struct BatchArgs {  // of k_resident_batch
+  const WholeOp* ops;
+  const WholeItem* items;
+  WholeCtl c;
+};
+
+// One tile, or two, per workgroup.  The workgroups of a region have
+// consecutive block indices, and workgroups start in that order on each XCD,
+// so those of the earliest unfinished region all run as soon as that many are
+// resident, which the planner keeps to half of the chip's room.  Launches of
+// resident passes of one process follow each other (the runtime chains them),
+// so no two share that room, nor the words.  Where the room is short all the
+// same (other processes), regions are called off and moved alone.
+template <int WL, bool MULTI, int ND, bool PAIR>
+__global__ __launch_bounds__(1024) void k_resident(WholeGeom g, char* data, WholeCtl c) {
+  extern __shared__ __align__(16) unsigned char lds[];
+  const uint32_t b = g.fwgs.div(blockIdx.x);
+  if (resident_body<WL, MULTI, ND, PAIR>(g, data, b, blockIdx.x - b * g.wgs, b, c, lds)) {
+    Const<ResidentArgs>* a = late((Const<ResidentArgs>*)__builtin_amdgcn_kernarg_segment_ptr());
+    finish_alone<WL>(&a->g, &a->c, a->data, b, b, lds);
+  }
+}
+
+// The same over the regions of many tensors: workgroup i takes item i.
 __global__ __launch_bounds__(kWholeBatchThreads) void k_resident_batch(const WholeOp* __restrict__ ops,
                                                         const WholeItem* __restrict__ items,
                                                         WholeCtl c) {
@@ -338,9 +384,10 @@ __global__ __launch_bounds__(kWholeBatchThreads) void k_resident_batch(const Who
   const WholeItem i = items[blockIdx.x];
   const WholeOp& o = ops[i.op];
   const WholeGeom& g = o.g;
+  bool alone = false;
 #define EH_WHOLE(WL, MULTI, ND)                                                       \
   case (WL)*4 + (MULTI)*2 + (ND == 4):                                                \
-    resident_body<WL, MULTI, ND, true>(g, o.data, i.b, i.t, i.slot, c, lds);          \
+    alone = resident_body<WL, MULTI, ND, true>(g, o.data, i.b, i.t, i.slot, c, lds);  \
     break;
 #define EH_WHOLE_W(WL)                                                                \
   EH_WHOLE(WL, false, 4) EH_WHOLE(WL, true, 4) EH_WHOLE(WL, false, 8) EH_WHOLE(WL, true, 8)
@@ -351,12 +398,23 @@ __global__ __launch_bounds__(kWholeBatchThreads) void k_resident_batch(const Who
     EH_WHOLE_W(3)
     EH_WHOLE_W(4)
   }
+  if (!alone) return;
+  Const<BatchArgs>* ka = late((Const<BatchArgs>*)__builtin_amdgcn_kernarg_segment_ptr());
+  Const<WholeOp>* op = (Const<WholeOp>*)(ka->ops + i.op);
+  switch (op->variant >> 2) {
+    case 0: finish_alone<0>(&op->g, &ka->c, op->data, i.b, i.slot, lds); break;
+    case 1: finish_alone<1>(&op->g, &ka->c, op->data, i.b, i.slot, lds); break;
+    case 2: finish_alone<2>(&op->g, &ka->c, op->data, i.b, i.slot, lds); break;
+    case 3: finish_alone<3>(&op->g, &ka->c, op->data, i.b, i.slot, lds); break;
+    case 4: finish_alone<4>(&op->g, &ka->c, op->data, i.b, i.slot, lds); break;
+  }
 #undef EH_WHOLE_W
 #undef EH_WHOLE
 }
 
-// the words of a device's resident passes over single tensors
-__device__ uint32_t g_ctl[whole_ctl_words(kWholeRegions)];
+// the words of a device's resident passes over single tensors, after those
+// of all its resident passes (each on a line of its own)
+__device__ uint32_t g_ctl[64 + whole_ctl_words(kWholeRegions)];
 
 // ---------------------------------------------------------------------------
 // orbit form
@@ -461,7 +519,10 @@ hipError_t launch_whole(const WholePass& p, char* data, const WholeCtl& ctl, hip
 hipError_t whole_ctl_device(WholeCtl& c) {
   void* p = nullptr;
   const hipError_t e = hipGetSymbolAddress(&p, HIP_SYMBOL(g_ctl));
-  if (e == hipSuccess) whole_ctl_at(c, (uint32_t*)p, kWholeRegions);
+  if (e != hipSuccess) return e;
+  c.recent = (uint32_t*)p;
+  c.lock = (uint32_t*)p + 32;
+  whole_ctl_at(c, (uint32_t*)p + 64, kWholeRegions);
   return e;
 }
 

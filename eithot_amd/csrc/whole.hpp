@@ -14,7 +14,8 @@
 //  * resident (WHOLE_RESIDENT): the tensor is a batch of regions, each small
 //    enough that all its tiles are held in the LDS of the chip at once.  The
 //    region's workgroups load their tiles, meet at a counter in device
-//    memory, and store.
+//    memory, and store.  Where they do not meet (the chip is shared), none
+//    stores and the last one moves the region alone.
 //
 // This header holds the geometry and the index arithmetic, shared by the
 // kernels, the planner and the CPU tests.
@@ -62,6 +63,7 @@ struct WholeGeom {
   uint32_t sg = 0, sna = 1, slast = 1;  // sna: tiles along dim 0
   FD32 fsgroup, fsg, fslast;
   uint64_t region = 0, B = 1;              // bytes per region, regions
+  uint32_t od[kWholeDims], ogin[kWholeDims];  // resident: extents and gin in output order
 };
 
 struct WholePass {
@@ -211,23 +213,108 @@ EH_HD uint32_t whole_elem(const WholeGeom& g, uint32_t p) {
   return l;
 }
 
-// Where resident passes meet: per region kWholeSubs counters, a root counter
-// (zero between passes) and a word that the region's last workgroup steps.
+// Byte offset in a region's input layout of element o of its output layout
+// (r dims; WholeGeom's od and ogin).
+EH_HD uint32_t whole_source(uint32_t r, const uint32_t* od, const uint32_t* ogin, uint32_t o) {
+  uint32_t a = 0;
+#pragma unroll
+  for (int k = 0; k < kWholeDims; ++k)
+    if (k < (int)r) {
+      const uint32_t q = o / od[k];
+      a += (o - q * od[k]) * ogin[k];
+      o = q;
+    }
+  return a;
+}
+
+// ---------------------------------------------------------------------------
+// Meeting of a region's workgroups.
+//
+// The workgroups that load a region must all be on the chip before one of
+// them may store.  Nothing guarantees that: other processes' workgroups, or a
+// stream that sees part of the chip, can keep the missing ones out for as
+// long as the present ones wait.  So a wait is bounded, and ends in ONE
+// decision for the region, taken by a compare-and-swap on its word: either
+// the last workgroup to arrive opens the region and all of them store, or one
+// that has waited long enough calls the pass off and none of them does.  All
+// workgroups still arrive once (those that start later too), and the last
+// one to arrive at a region called off finds it as it was, with everybody
+// else gone or leaving, and moves it alone through host memory.
+//
+// Per region: kWholeSubs counters and a root counter (zero between passes)
+// and the word, 4 * passes + flags.  For all regions of a device: the time
+// of the last pass called off, for a while after which workgroups wait less
+// (what kept one region's workgroups apart keeps the next one's), and a lock
+// on the host memory.
+// ---------------------------------------------------------------------------
 constexpr uint32_t kWholeSubs = 16;
+constexpr uint32_t kCalledOff = 1;   // this pass of the region
+constexpr uint32_t kWasCalledOff = 2;  // the one before
 struct WholeCtl {
-  uint32_t* failed = nullptr;  // set by a workgroup that gave up waiting
   uint32_t *open = nullptr, *root = nullptr, *sub = nullptr;
-  uint32_t slots = 0;                // regions the words serve
-  uint64_t patience = 0;             // ticks of the 100 MHz clock
-  uint32_t* host_failed = nullptr;   // pinned host word, set along with *failed
+  uint32_t slots = 0;            // regions these words serve
+  uint32_t* recent = nullptr;    // time of the last pass called off, 2^20 ticks
+  uint32_t* lock = nullptr;      // 1: a workgroup uses `room`
+  char* room = nullptr;          // pinned host memory, as large as the largest region
+  uint64_t patience = 0;         // ticks of the 100 MHz clock
 };
-constexpr uint64_t whole_ctl_words(uint32_t slots) { return 32 + (uint64_t)slots * (2 + kWholeSubs); }
+constexpr uint64_t whole_ctl_words(uint32_t slots) { return (uint64_t)slots * (2 + kWholeSubs); }
 inline void whole_ctl_at(WholeCtl& c, uint32_t* words, uint32_t slots) {
-  c.failed = words;
-  c.open = words + 32;
+  c.open = words;
   c.root = c.open + slots;
   c.sub = c.root + slots;
   c.slots = slots;
+}
+
+enum WholeMeet : uint32_t { MEET_STORE = 0, MEET_LEAVE = 1, MEET_ALONE = 2 };
+
+// W gives the words: add, get, set, cas (true when it swapped), now (ticks),
+// pause.  The counters are spread (each on a line of its own: one address
+// takes about 30 ns per addition).
+template <class W>
+EH_HD bool whole_arrive(const WholeCtl& c, uint32_t slot, uint32_t t, uint32_t n) {
+  const uint32_t subs = n <= kWholeSubs ? 1 : kWholeSubs;
+  const uint32_t j = t % subs, members = (n - j + subs - 1) / subs;
+  uint32_t* sub = c.sub + (uint64_t)j * c.slots + slot;
+  if (W::add(sub, 1) != members - 1) return false;
+  W::set(sub, 0);
+  if (subs == 1) return true;
+  if (W::add(c.root + slot, 1) != subs - 1) return false;
+  W::set(c.root + slot, 0);
+  return true;
+}
+
+// What workgroup t of the region's n does, having loaded its part; `word` is
+// the region's word as it was before it arrived.
+template <class W>
+EH_HD WholeMeet whole_meet(const WholeCtl& c, uint32_t slot, uint32_t t, uint32_t n, uint32_t word) {
+  uint32_t* open = c.open + slot;
+  if (whole_arrive<W>(c, slot, t, n))
+    return !(word & kCalledOff) && W::cas(open, word, (word | 3) + 1) ? MEET_STORE : MEET_ALONE;
+  if (word & kCalledOff) return MEET_LEAVE;
+  const uint64_t t0 = W::now();
+  // a second after a pass was called off: 1 ms at most
+  const bool soon = (uint32_t)(t0 >> 20) - W::get(c.recent) < 96;
+  const uint64_t patience = soon && c.patience > 100000 ? 100000 : c.patience;
+  for (;;) {
+    const uint32_t now = W::get(open);
+    if ((now | 3) != (word | 3)) return now & kWasCalledOff ? MEET_LEAVE : MEET_STORE;
+    if (now & kCalledOff) return MEET_LEAVE;
+    if (W::now() - t0 > patience) {
+      if (W::cas(open, word, word | kCalledOff)) {
+        W::set(c.recent, (uint32_t)(W::now() >> 20));
+        return MEET_LEAVE;
+      }
+    } else {
+      W::pause();
+    }
+  }
+}
+
+// Ends a pass that MEET_ALONE's workgroup has done.
+template <class W>
+EH_HD void whole_done_alone(uint32_t* open, uint32_t word) {
+  W::set(open, ((word | 3) + 1) | kWasCalledOff);
 }
 
 // Plans the whole-permutation pass of a tensor (perm1 1-based) for a chip of

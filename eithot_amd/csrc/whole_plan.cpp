@@ -155,6 +155,8 @@ bool build(const Canon& c, const std::vector<int64_t>& t, WholeGeom& g) {
     g.oft[k].init(g.t[a]);
     g.ols[k] = g.ls[a];
     g.ogout[k] = g.gout[a];
+    g.od[k] = g.d[a];
+    g.ogin[k] = (uint32_t)g.gin[a];
   }
   // offsets within a tile stay below 4 GB (a 16-byte access past them too)
   unsigned __int128 sin = 64, sout = 64;
@@ -302,8 +304,8 @@ WholePass plan_whole(const int64_t* dims, const int* perm1, int rank, size_t ele
   // registers, for larger ones and batches (210 MB in regions of 3.6 MB:
   // 158 -> 100 us; one tile each 114, 32 KiB tiles 99, but 38 instead of 43 us
   // for 52 MB of bytes and 121 instead of 117 for 236 MB; 128 KiB 130).  A
-  // region takes at most half of the workgroups the chip holds, so
-  // that two processes can always run theirs.
+  // region takes at most half of the workgroups the chip holds: the others'
+  // room is for what else runs, so that its workgroups meet soon.
   if (c.B <= (int64_t)kWholeRegions) {
     std::vector<int> cls(r);
     for (int k = 0; k < r; ++k) cls[k] = k;

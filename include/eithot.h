@@ -255,6 +255,12 @@ int eithot_plan_segments(const int64_t* dims, const int* perm, int order, size_t
  *                    chip's LDS holds whole), instead of the plan's passes (1;
  *                    0: never).  Off while any knob of the passes differs
  *                    from its default
+ *   "whole_patience" microseconds (100000; 0 to 60000000) that the workgroups of
+ *                    such a region wait for each other.  Where other work
+ *                    keeps them apart for longer, the region is moved through
+ *                    pinned host memory by one workgroup (1 to 64 MiB, as
+ *                    large as the largest region): slowly, with the same
+ *                    result.  A batch keeps the value it was built with
  *   "hold_floor"     device bytes (arena and pass tables) the library may keep
  *                    after a call even when alpha * tensor bytes is smaller
  *                    (64 MiB; 0: alpha alone bounds them)
