@@ -5,6 +5,7 @@
 #include <algorithm>
 #include <cstdarg>
 #include <cstdio>
+#include <cstdlib>
 #include <cstring>
 #include <functional>
 #include <map>
@@ -239,10 +240,29 @@ bool stream_captured(hipStream_t stream) {
   return cap != hipStreamCaptureStatusNone;
 }
 
+// Whether work on `stream` may run on every CU: a region's workgroups are
+// counted against the whole chip.  The HIP runtime knows the masks of streams
+// and its own (which the null stream has), the one below it is asked for in
+// the environment.
+static bool sees_all_cus(int cus, hipStream_t stream) {
+  static const bool below = std::getenv("HSA_CU_MASK") != nullptr;
+  uint32_t mask[32] = {0};
+  const int words = (cus + 31) / 32;
+  if (below || words > 32) return false;
+  if (hipExtStreamGetCUMask(stream, (uint32_t)words, mask) != hipSuccess) {
+    (void)hipGetLastError();
+    return false;
+  }
+  int n = 0;
+  for (int k = 0; k < words; ++k) n += __builtin_popcount(mask[k]);
+  return n >= cus;
+}
+
 bool Device::takes_whole_locked(const Plan& plan, hipStream_t stream) {
   if (!plan.whole) return false;
   if (plan.whole->mode == WHOLE_ORBIT) return true;
-  return !stream_captured(stream) && whole_begin_locked(plan.whole->g.region, stream);
+  return !stream_captured(stream) && sees_all_cus(prof.cus, stream) &&
+         whole_begin_locked(plan.whole->g.region, stream);
 }
 
 bool Device::whole_room_locked(uint64_t region) {

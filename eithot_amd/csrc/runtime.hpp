@@ -79,7 +79,8 @@ struct Device {
 
   // With enqueue_mu held: whether a call of `plan` on `stream` runs its
   // whole-permutation pass, which run_plan then launches.  Resident passes
-  // are left out of stream captures (a replay could not be chained).
+  // are left out of stream captures (a replay could not be chained) and of
+  // streams that see part of the chip.
   bool takes_whole_locked(const Plan& plan, hipStream_t stream);
   // Resident passes over regions of up to `region` bytes on `stream` go
   // between these two (false: the device or the stream can run none now);

@@ -254,7 +254,8 @@ int eithot_plan_segments(const int64_t* dims, const int* perm, int order, size_t
  *                    same in input and output order, or regions that the
  *                    chip's LDS holds whole), instead of the plan's passes (1;
  *                    0: never).  Off while any knob of the passes differs
- *                    from its default
+ *                    from its default; regions need a stream that sees the
+ *                    whole chip and is not captured
  *   "whole_patience" microseconds (100000; 0 to 60000000) that the workgroups of
  *                    such a region wait for each other.  Where other work
  *                    keeps them apart for longer, the region is moved through
