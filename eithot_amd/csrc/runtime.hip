@@ -261,8 +261,7 @@ static bool sees_all_cus(int cus, hipStream_t stream) {
 bool Device::takes_whole_locked(const Plan& plan, hipStream_t stream) {
   if (!plan.whole) return false;
   if (plan.whole->mode == WHOLE_ORBIT) return true;
-  return !stream_captured(stream) && sees_all_cus(prof.cus, stream) &&
-         whole_begin_locked(plan.whole->g.region, stream);
+  return sees_all_cus(prof.cus, stream) && whole_begin_locked(plan.whole->g.region, stream);
 }
 
 bool Device::whole_room_locked(uint64_t region) {
@@ -292,7 +291,9 @@ bool Device::whole_room_locked(uint64_t region) {
 // recorded behind them only when a call on another stream needs it (the null
 // stream outlives every call, other streams may not).
 bool Device::whole_begin_locked(uint64_t region, hipStream_t stream) {
-  if (!whole_room_locked(region)) return false;
+  // (an event waited for or recorded on a captured stream would draw the
+  // streams of later passes into the capture)
+  if (stream_captured(stream) || !whole_room_locked(region)) return false;
   if (!stream && !whole_elsewhere) return true;
   if ((!whole_elsewhere && hipEventRecord(whole_ready, nullptr) != hipSuccess) ||
       hipStreamWaitEvent(stream, whole_ready, 0) != hipSuccess) {

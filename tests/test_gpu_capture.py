@@ -129,3 +129,44 @@ def test_capture_mode_is_left_as_it_was(torch_cuda):
             x.check(f"replay {k}")
             y.check(f"replay {k}")
         g.close()
+
+
+def test_batch_run_on_a_captured_stream(torch_cuda):
+    # the batch's own graph is launched, not captured, and resident passes of
+    # other streams, during the capture and after it, are no part of it either
+    torch = torch_cuda
+    a, b, c = (Case(torch, [1021, 523], [2, 1], 4, k) for k in (11, 12, 13))
+    batch = E.Batch()
+    batch.add(a.buf.data_ptr(), a.dims, a.perm, a.elem)
+    batch.add(b.buf.data_ptr(), b.dims, b.perm, b.elem)
+    batch.build()
+    side = torch.cuda.Stream()
+    c.call(side.cuda_stream)
+    torch.cuda.synchronize()
+    for k in range(3):
+        for x in (a, b, c):
+            x.buf.copy_(x.src)
+        torch.cuda.synchronize()
+
+        def calls(stream):
+            batch.run(stream=stream, sync=False)
+            c.call(side.cuda_stream)
+
+        print(f"batch on a captured stream {k}", flush=True)
+        g = Graph(calls)
+        nodes = g.nodes
+        g.close()
+        torch.cuda.synchronize()
+        assert nodes == 0
+        c.check(f"during {k}")
+        c.buf.copy_(c.src)
+        torch.cuda.synchronize()
+        c.call(None if k else side.cuda_stream)
+        torch.cuda.synchronize()
+        c.check(f"after {k}")
+        a.buf.copy_(a.src)
+        b.buf.copy_(b.src)
+        torch.cuda.synchronize()
+        batch.run()
+        a.check(f"batch {k}")
+        b.check(f"batch {k}")
