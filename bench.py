@@ -216,7 +216,7 @@ def run_single(name, dims, perm, elem, alpha, mode, seed, steps):
         n = E.lib().eithot_last_pass_times(None, 0)
         arr = (ctypes.c_float * n)()
         E.lib().eithot_last_pass_times(arr, n)
-        passes.append((k % 2, list(arr)))
+        passes.append((k % 2, list(arr), E.last_whole_pass()))
         peak = max(peak, E.last_peak_extra_bytes())
         print(f"bench {name}: step {k} {times[-1] * 1e3:.2f} ms", file=sys.stderr, flush=True)
         if k == 0:
@@ -243,9 +243,9 @@ def run_single(name, dims, perm, elem, alpha, mode, seed, steps):
     fwd = [t for k, t in enumerate(times) if k % 2 == 0]
     t = sorted(fwd)[len(fwd) // 2]
     ops, _ = E.plan_describe(dims, perm, elem, 1, alpha)
-    fwd_pass = [p for w, p in passes if w == 0]
+    fwd_pass = [p for w, p, _ in passes if w == 0]
     per_pass = []
-    if len(fwd_pass[0]) < len(ops):  # one whole pass did the work of all of them
+    if passes[0][2]:  # one whole pass did the work of all of them
         ms = sorted(x[0] for x in fwd_pass)[len(fwd_pass) // 2]
         per_pass.append({"kernel": "whole", "ms": round(ms, 4),
                          "GBps_2x_tensor": round(2 * nbytes / (ms / 1e3) / 1e9, 1)})
@@ -449,6 +449,7 @@ def run_census(which="serve", count=None):
         E.transpose_tensor(buf, dims, perm, elem, 1, 0.05)  # plans; tables uploaded
         E.fill_pattern(buf, vol, elem, 5000 + k, 1)
         E.transpose_tensor(buf, dims, perm, elem, 1, 0.05)
+        whole = E.last_whole_pass()
         n = E.lib().eithot_last_pass_times(None, 0)
         arr = (ctypes.c_float * n)()
         E.lib().eithot_last_pass_times(arr, n)
@@ -456,8 +457,7 @@ def run_census(which="serve", count=None):
             print(f"census: request {k} {dims} {perm} differs", file=sys.stderr)
             sys.exit(1)
         ops, _ = E.plan_describe(dims, perm, elem, 1, 0.05)
-        classes = ([pass_class(op, buf.data_ptr()) for op in ops] if len(arr) == len(ops)
-                   else ["whole"])
+        classes = ["whole"] if whole else [pass_class(op, buf.data_ptr()) for op in ops]
         for name, ms in zip(classes, arr):
             c = agg.setdefault(name, {"passes": 0, "ms": 0.0, "bytes": 0})
             c["passes"] += 1
@@ -557,6 +557,7 @@ def measure(spec, steps, warmup, label):
           flush=True)
     E.lib().eithot_set_pass_timing(1)
     pass_ms = {0: [], 1: []}
+    whole = {}
     peak = 0
     torch.cuda.synchronize()
     t0 = time.perf_counter()
@@ -566,6 +567,7 @@ def measure(spec, steps, warmup, label):
         arr = (ctypes.c_float * n)()
         E.lib().eithot_last_pass_times(arr, n)
         pass_ms[i % 2].append(list(arr))
+        whole[i % 2] = E.last_whole_pass()
         peak = max(peak, E.last_peak_extra_bytes())
     torch.cuda.synchronize()
     elapsed = time.perf_counter() - t0
@@ -589,12 +591,13 @@ def measure(spec, steps, warmup, label):
         if not times:
             continue
         ops, _ = E.plan_describe(cases[which][0], cases[which][1], elem, n_sub, alpha)
+        names = ["whole"] if whole[which] else [kernel_name(op) for op in ops]
         passes["forward" if which == 0 else "inverse"] = [
-            {"kernel": kernel_name(op), "ms": round(sum(t[k] for t in times) / len(times), 4)}
-            for k, op in enumerate(ops)]
-        for k, op in enumerate(ops):
+            {"kernel": name, "ms": round(sum(t[k] for t in times) / len(times), 4)}
+            for k, name in enumerate(names)]
+        for k, name in enumerate(names):
             ms = sum(t[k] for t in times) / len(times)
-            a = agg.setdefault(kernel_name(op), {"ms": 0.0, "launches": 0})
+            a = agg.setdefault(name, {"ms": 0.0, "launches": 0})
             a["ms"] += ms
             a["launches"] += 1
     for v in agg.values():

@@ -21,7 +21,8 @@ from . import _lib
 from ._lib import EithotError, check, i32, i64, lib
 
 __all__ = ["transpose", "transpose_tensor", "transpose_ptr", "estimate", "estimate_reference",
-           "decompose", "plan_describe", "plan_partition", "last_peak_extra_bytes", "fill_pattern",
+           "decompose", "plan_describe", "plan_partition", "last_peak_extra_bytes", "last_whole_pass",
+           "fill_pattern",
            "verify_pattern", "set_tuning", "get_tuning", "Batch", "Server", "EithotError"]
 
 
@@ -68,6 +69,11 @@ def transpose_tensor(t, dims, perm1, elem_bytes=None, n_sub=1, alpha=0.05, strea
 
 def last_peak_extra_bytes():
     return int(lib().eithot_last_peak_extra_bytes())
+
+
+def last_whole_pass():
+    """0 if this thread's last transpose ran its plan's passes, else the whole pass's form (1, 2)."""
+    return int(lib().eithot_last_whole_pass())
 
 
 def estimate(dims, perm1, elem_bytes, alpha):

@@ -26,7 +26,7 @@ ERRORS = {
 EXPORTS = [
     "eithot_transpose", "eithot_transpose_async", "eithot_transpose_noalloc",
     "eithot_inplace_transpose",
-    "eithot_last_peak_extra_bytes", "eithot_last_error", "eithot_release", "eithot_estimate",
+    "eithot_last_peak_extra_bytes", "eithot_last_whole_pass", "eithot_last_error", "eithot_release", "eithot_estimate",
     "eithot_estimate_reference", "eithot_decompose", "eithot_plan_describe",
     "eithot_plan_partition", "eithot_plan_block_table", "eithot_plan_cycle_maps",
     "eithot_plan_segments",

@@ -90,6 +90,7 @@ using namespace eithot;
 extern "C" int eithot_transpose_noalloc(void* dev, const int64_t* dims, const int* perm, int order,
                                         size_t elem_bytes, int n_sub, double alpha) {
   set_peak(0);
+  set_whole(WHOLE_NONE);
   int rc = validate(dev, dims, perm, order, elem_bytes);
   if (rc) return rc;
   if (!(alpha > 0)) return fail(EITHOT_ERR_INVALID, "alpha must be > 0");

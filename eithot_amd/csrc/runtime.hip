@@ -26,6 +26,7 @@ namespace eithot {
 namespace {
 thread_local std::string g_err;
 thread_local size_t g_peak = 0;
+thread_local int g_whole = 0;
 thread_local std::vector<float> g_pass_ms;
 int g_timing = 0;
 }  // namespace
@@ -41,6 +42,7 @@ int fail(int code, const char* fmt, ...) {
 }
 
 void set_peak(size_t b) { g_peak = b; }
+void set_whole(int mode) { g_whole = mode; }
 
 Device* device_ctx(int* err) {
   static std::mutex mu;
@@ -434,6 +436,7 @@ int run_plan(Device* d, const Plan& plan, char* data, char* scratch, int64_t scr
   }
   int rc = EITHOT_OK;
   const size_t npass = whole ? 1 : plan.ops.size();
+  set_whole(whole ? plan.whole->mode : WHOLE_NONE);
   if (whole) {
     const hipError_t e = launch_whole(*plan.whole, data, d->whole_ctl, stream);
     if (e != hipSuccess)
@@ -619,6 +622,7 @@ static int transpose_impl(void* dev, const int64_t* dims, const int* perm, int o
                           int n_sub, double alpha, hipStream_t stream, bool sync) {
   g_err.clear();
   g_peak = 0;
+  g_whole = WHOLE_NONE;
   int rc = validate(dev, dims, perm, order, elem);
   if (rc) return rc;
   if (!(alpha > 0)) return fail(EITHOT_ERR_INVALID, "alpha must be > 0");
@@ -707,6 +711,8 @@ int eithot_inplace_transpose(void* data, int source, int rank, const int* dim,
 }
 
 size_t eithot_last_peak_extra_bytes(void) { return g_peak; }
+
+int eithot_last_whole_pass(void) { return g_whole; }
 
 const char* eithot_last_error(void) { return g_err.c_str(); }
 

@@ -98,6 +98,7 @@ std::string plan_key(const int64_t* dims, const int* perm1, int rank, size_t ele
 Device* device_ctx(int* err);
 int fail(int code, const char* fmt, ...);
 void set_peak(size_t bytes);
+void set_whole(int mode);
 int validate(const void* dev, const int64_t* dims, const int* perm, int order, size_t elem);
 // Enqueues the plan's passes on `stream`.  min_groups_cap > 0 lowers the
 // launch configuration's workgroup floor per pass to at most that (callers

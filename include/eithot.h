@@ -99,6 +99,11 @@ int eithot_inplace_transpose(void* data, int source, int rank, const int* dim,
  * counted. */
 size_t eithot_last_peak_extra_bytes(void);
 
+/* How the calling thread's last transpose ran: 0 the plan's passes, 1 or 2
+ * one whole pass (tuning key "whole") over lengths that read the same, or
+ * over regions. */
+int eithot_last_whole_pass(void);
+
 /* Message of the calling thread's last failure ("" if none). */
 const char* eithot_last_error(void);
 
