@@ -1085,7 +1085,7 @@ constexpr const char* kPassKnobs[] = {
     "fuse_max_block", "block_digits",   "block_pad",       "cycle_word_cost", "threads",
     "threads_big",    "xcd_remap",      "cycle_variant",   "reorder",         "regroup",
     "cycle_lmax",     "cycle_cell_pref", "segtile_threads", "lds_threads_auto", "segtile_nt",
-    "lower_mask",     "cycle_u_depth",  "min_groups"};
+    "lower_mask",     "min_groups"};
 
 int tuning_set(const char* key, int64_t value) {
   std::lock_guard<std::mutex> lk(g_tune_mu);

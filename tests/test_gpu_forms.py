@@ -24,3 +24,13 @@ def test_form_is_told(torch_cuda, dims, perm, elem, form):
             E.set_tuning("whole", old)
         assert np.array_equal(got, want)
         assert E.last_whole_pass() == (form if whole else 0)
+
+
+def test_knob_without_effect_leaves_the_form(torch_cuda):
+    for value in (6, 8):
+        old = E.set_tuning("cycle_u_depth", value)
+        try:
+            run_case(torch_cuda, [500, 500], [2, 1], 4)
+        finally:
+            E.set_tuning("cycle_u_depth", old)
+        assert E.last_whole_pass() == 1
