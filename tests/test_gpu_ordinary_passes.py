@@ -20,5 +20,4 @@ pytestmark = pytest.mark.gpu
 def ordinary_passes():
     old = E.set_tuning("whole", 0)
     yield
-    E.set_tuning("whole", old)
-    assert E.last_whole_pass() == 0
+    assert E.set_tuning("whole", old) == 0
