@@ -354,9 +354,28 @@ void walk_parallel(const Src& src, uint64_t N, int64_t lmax, std::vector<uint64_
 }
 }  // namespace
 
+// Segments of short cycles grouped by length in steps of 8 (the kernel's
+// unrolled step), longest first, each group in its own order (a counting
+// sort, so neighbouring starts stay neighbours): cells under 1 KiB share a
+// wave, which runs until its longest segment ends.  A 207 MB pass of 128-byte
+// cells with cycles of 1 to 60 positions: 126 -> 122 us.  Long cycles, cut
+// into nearly equal segments, keep their order, which the grouping disturbs
+// (4.5 GB, 128-byte cells: 2 % slower with it).
+static void group_by_length(CycleTable& t) {
+  if (t.mean > 32) return;
+  constexpr uint32_t kGroups = 33;  // the last takes every length above 256
+  auto group = [](const CycleSeg& s) { return kGroups - 1 - std::min((s.len - 1) / 8, kGroups - 1); };
+  std::vector<size_t> at(kGroups + 1, 0);
+  for (const CycleSeg& s : t.segs) ++at[group(s) + 1];
+  for (uint32_t g = 0; g < kGroups; ++g) at[g + 1] += at[g];
+  std::vector<CycleSeg> sorted(t.segs.size());
+  for (const CycleSeg& s : t.segs) sorted[at[group(s)]++] = s;
+  t.segs.swap(sorted);
+}
+
 std::shared_ptr<CycleTable> build_cycle_table_maps(const std::vector<CycleMap>& maps, int64_t N,
-                                                   int64_t lmax) {
-  std::vector<int64_t> key = {N, lmax};
+                                                   int64_t lmax, bool by_length) {
+  std::vector<int64_t> key = {N, lmax, by_length};
   for (const CycleMap& M : maps) key.insert(key.end(), {M.bc, M.R, M.C, M.m});
   {
     std::lock_guard<std::mutex> lk(g_cyc_mu);
@@ -414,6 +433,10 @@ std::shared_ptr<CycleTable> build_cycle_table_maps(const std::vector<CycleMap>& 
       t->segs.push_back({starts[i], (uint32_t)len, (int32_t)(first_slot + (i + 1) % n), 0});
     }
   }
+  t->mean = t->mean_len();
+  if (by_length) group_by_length(*t);
+  cycle_digits(*t, N);
+  // final from here on: other plans share it, in other threads too
   std::lock_guard<std::mutex> lk(g_cyc_mu);
   if (g_cyc_cache.size() >= 16) g_cyc_cache.clear();
   g_cyc_cache[key] = t;
@@ -700,35 +723,17 @@ std::shared_ptr<CycleTable> choose_cycle_table(const std::vector<CycleMap>& maps
                                                int64_t lmax0) {
   const int64_t chunk = 64 * pow2_factor(U, 16);
   const int64_t chunks = (U + chunk - 1) / chunk;
+  const bool by_length = U < 1024;
   int64_t lmax = lmax0 > 0 ? lmax0 : 256;
-  std::shared_ptr<CycleTable> t = build_cycle_table_maps(maps, N, lmax);
+  std::shared_ptr<CycleTable> t = build_cycle_table_maps(maps, N, lmax, by_length);
   while (!lmax0 && lmax > 16 && B * (int64_t)t->segs.size() * chunks < 32768) {
     lmax /= 2;
-    t = build_cycle_table_maps(maps, N, lmax);
+    t = build_cycle_table_maps(maps, N, lmax, by_length);
   }
   while (!t->slots.empty() && B * (int64_t)t->slots.size() * U + t->bytes() > budget) {
     lmax = lmax >= N ? N : lmax * 2;
-    t = build_cycle_table_maps(maps, N, lmax);
+    t = build_cycle_table_maps(maps, N, lmax, by_length);
   }
-  // Cells under 1 KiB share a wave, which runs until its longest segment
-  // ends: segments of short cycles are grouped by length in steps of 8 (the
-  // kernel's unrolled step), longest first, each group in its own order (a
-  // counting sort, so neighbouring starts stay neighbours).  A 207 MB pass
-  // of 128-byte cells with cycles of 1 to 60 positions: 126 -> 122 us.  Long
-  // cycles, cut into nearly equal segments, keep their order, which the
-  // grouping disturbs (4.5 GB, 128-byte cells: 2 % slower with it).
-  t->mean = t->mean_len();
-  if (U < 1024 && t->mean <= 32) {
-    constexpr uint32_t kGroups = 33;  // the last takes every length above 256
-    auto group = [](const CycleSeg& s) { return kGroups - 1 - std::min((s.len - 1) / 8, kGroups - 1); };
-    std::vector<size_t> at(kGroups + 1, 0);
-    for (const CycleSeg& s : t->segs) ++at[group(s) + 1];
-    for (uint32_t g = 0; g < kGroups; ++g) at[g + 1] += at[g];
-    std::vector<CycleSeg> sorted(t->segs.size());
-    for (const CycleSeg& s : t->segs) sorted[at[group(s)]++] = s;
-    t->segs.swap(sorted);
-  }
-  cycle_digits(*t, N);
   return t;
 }
 

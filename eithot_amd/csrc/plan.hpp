@@ -110,7 +110,7 @@ struct CycleTable {
     for (const CycleSeg& s : segs) n += s.len;
     return segs.empty() ? 0 : (uint32_t)((n + segs.size() - 1) / segs.size());
   }
-  uint32_t mean = 0;  // mean_len(), set once the table is final
+  uint32_t mean = 0;  // mean_len()
   int64_t bytes() const { return (int64_t)(segs.size() * sizeof(CycleSeg) + slots.size() * 4); }
   // device copies (segs then slots), one per device id, made by the launcher
   DeviceCopies dev;
@@ -143,8 +143,10 @@ void cycle_digits(CycleTable& t, int64_t N);
 // Builds the table (fixed points are skipped).  R*C must be below 2^32.
 std::shared_ptr<CycleTable> build_cycle_table(int64_t R, int64_t C, int64_t lmax);
 // Same over the composition of several cell maps on N cells (N < 2^32).
+// by_length: short segments grouped by their length.  Tables are cached and
+// shared: nothing but their device copies changes afterwards.
 std::shared_ptr<CycleTable> build_cycle_table_maps(const std::vector<CycleMap>& maps, int64_t N,
-                                                   int64_t lmax);
+                                                   int64_t lmax, bool by_length = false);
 
 // Gather table of a fused block permutation (OP_BLOCK): consecutive
 // contiguous tile passes whose matrices nest inside blocks of `cells` cells
