@@ -11,6 +11,7 @@
 #include <sstream>
 #include <thread>
 #include <tuple>
+#include <unordered_map>
 
 #include "eithot_status.h"
 
@@ -605,7 +606,7 @@ CatPlan plan_catanzaro(int64_t R, int64_t C, int64_t U, const DeviceProfile& pro
 }
 
 const std::vector<int64_t>& divisors(int64_t x) {
-  thread_local std::map<int64_t, std::vector<int64_t>> memo;
+  thread_local std::unordered_map<int64_t, std::vector<int64_t>> memo;
   auto it = memo.find(x);
   if (it != memo.end()) return it->second;
   if (memo.size() > 4096) memo.clear();
@@ -794,8 +795,9 @@ thread_local bool g_cycle_small = false;      // cycle passes may move small cel
 // 357-456, 20-24 bytes 607-671, 16 bytes 887; from 64 bytes 0.15 more, against
 // plans that would only tie.
 constexpr uint64_t kCycleMaxSmallCells = 1ull << 23;  // planned in 0.2-0.35 s
+constexpr double kCostSmallCells = 1.8;  // the least of them
 inline double small_cycle_cost(int64_t U) {
-  if (U >= 64) return U % 64 ? 2.05 : 1.8;
+  if (U >= 64) return U % 64 ? 2.05 : kCostSmallCells;
   return U >= 32 ? 3.3 : U > 16 ? 5.5 : 7.4;
 }
 // What a column or row pass of such cells takes beyond cat_pass_cost, in the
@@ -837,7 +839,22 @@ struct Choice {
 struct Lowerer {
   const DeviceProfile& prof;
   int64_t scratch_budget;
-  std::map<std::tuple<int64_t, int64_t, int64_t, int>, Choice> memo;
+  struct Key {
+    int64_t R, C, U;
+    bool operator==(const Key& o) const { return R == o.R && C == o.C && U == o.U; }
+  };
+  struct KeyHash {
+    size_t operator()(const Key& k) const {
+      uint64_t h = (uint64_t)k.R * 0x9E3779B97F4A7C15ull;
+      h = (h ^ (h >> 29) ^ (uint64_t)k.C) * 0xBF58476D1CE4E5B9ull;
+      h = (h ^ (h >> 32) ^ (uint64_t)k.U) * 0x94D049BB133111EBull;
+      return (size_t)(h ^ (h >> 31));
+    }
+  };
+  std::unordered_map<Key, Choice, KeyHash> memo;
+  // of a search with cycle passes of small cells: the search without, whose
+  // choices for larger cells are the same
+  const Lowerer* plain = nullptr;
 
   Lowerer(const DeviceProfile& p, int64_t budget) : prof(p), scratch_budget(budget) {}
 
@@ -848,9 +865,13 @@ struct Lowerer {
       ch.cost = 0;
       return ch;
     }
-    auto key = std::make_tuple(R, C, U, 0);  // first result wins at any depth
+    const Key key{R, C, U};  // first result wins at any depth
     auto it = memo.find(key);
     if (it != memo.end()) return it->second;
+    if (plain && U >= prof.cycle_min_cell) {
+      auto old = plain->memo.find(key);
+      if (old != plain->memo.end()) return old->second;
+    }
     const int64_t mask = prof.lower_mask;
     if (int64_t us = (mask & LOWER_TILE) ? pick_tile_slice(R, C, U, prof) : 0) {
       ch.how = HOW_TILE;
@@ -1990,11 +2011,17 @@ static int make_plan_search(const int64_t* dims_in, const int* perm1, int rank, 
   Regroup rg;
   const bool regroup = vol_ok && !partition && reorder == 0 && prof.regroup &&
                        rg.canonical(dims_in, perm1, rank, elem) && rg.q.size() >= 3;
+  DeviceProfile profs[2] = {prof, prof};
+  profs[0].staged_mult = 1.0;
+  profs[1].staged_mult = 3.0;
+  Lowerer plain[2] = {{profs[0], budget0}, {profs[1], budget0}};
   auto search = [&] {
-    for (double mult : {1.0, 3.0}) {
-      DeviceProfile p2 = prof;
-      p2.staged_mult = mult;
-      Lowerer shared(p2, budget0);
+    for (int m : {0, 1}) {
+      const DeviceProfile& p2 = profs[m];
+      const double mult = p2.staged_mult;
+      Lowerer cells(p2, budget0);
+      cells.plain = &plain[m];
+      Lowerer& shared = g_cycle_small ? cells : plain[m];
       for (int o : orders) {
         Plan q;
         const int r =
@@ -2041,8 +2068,15 @@ static int make_plan_search(const int64_t* dims_in, const int* perm1, int rank, 
   g_cycle_small = false;
   search();
   if (rc) return rc;
-  // again with cycle passes of small cells, kept where they cost less
-  if (small && g_cycle_shift) {
+  // Again with cycle passes of small cells, kept where they cost less, unless
+  // the plan costs less than any with one: that pass, and one more at least
+  // where the elements that stay together make no such cell.  First plans of
+  // 500 shapes took 8.1 s without this search, 10.3 s with a full one each
+  // time, and 8.6 s so, with the lowerer's memo hashed and shared.
+  Regroup together;
+  together.canonical(dims_in, perm1, rank, elem);
+  const double least = kCostSmallCells + (together.E < 16 ? kCostTile : 0.0);
+  if (small && g_cycle_shift && small_cell_cost(plan) > least) {
     Plan first = std::move(plan);
     const int order1 = best_order;
     const double mult1 = best_mult;

@@ -1,6 +1,8 @@
 // Host checks of the planner's cached pass tables (eithot_amd/csrc/plan.cpp)
 // for the CPU tests.  Compiled by the test with hipcc, never part of the
 // product.
+#include <chrono>
+
 #include "../eithot_amd/csrc/plan.cpp"
 
 using namespace eithot;
@@ -38,4 +40,19 @@ extern "C" int pt_replan(const int64_t* dims, const int* perm1, int rank, int64_
       return 1 + (int)i;
   }
   return 0;
+}
+
+// Shortest of `reps` planning times (ms), with or without cycle passes of small cells.
+extern "C" double pt_plan_ms(const int64_t* dims, const int* perm1, int rank, int64_t elem, int small,
+                             int reps) {
+  DeviceProfile prof;
+  prof.cycle_small = small;
+  double best = 1e300;
+  for (int k = 0; k < reps; ++k) {
+    Plan p;
+    const auto t0 = std::chrono::steady_clock::now();
+    if (make_plan(dims, perm1, rank, (size_t)elem, 1, 0.05, prof, 0, p)) return -1;
+    best = std::min(best, std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count());
+  }
+  return best;
 }

@@ -22,9 +22,11 @@ def pt():
                                "-std=c++17", "-fPIC", "-shared", "-pthread", "-o", tmp, src])
         os.replace(tmp, SO)
     L = ctypes.CDLL(SO)
-    L.pt_replan.argtypes = [ctypes.POINTER(ctypes.c_int64), ctypes.POINTER(ctypes.c_int),
-                            ctypes.c_int, ctypes.c_int64, ctypes.c_int64,
-                            ctypes.POINTER(ctypes.c_int)]
+    shape = [ctypes.POINTER(ctypes.c_int64), ctypes.POINTER(ctypes.c_int), ctypes.c_int,
+             ctypes.c_int64]
+    L.pt_replan.argtypes = shape + [ctypes.c_int64, ctypes.POINTER(ctypes.c_int)]
+    L.pt_plan_ms.argtypes = shape + [ctypes.c_int, ctypes.c_int]
+    L.pt_plan_ms.restype = ctypes.c_double
     return L
 
 
@@ -38,3 +40,12 @@ def test_tables_of_a_plan_stay(pt, dims, perm, elem, other):
                      len(dims), elem, other, ctypes.byref(n))
     assert r == 0, f"pass {r - 1}'s table changed"
     assert n.value > 0
+
+
+# plans that cost less than any with a pass of small cells could
+@pytest.mark.parametrize("dims,perm,elem", [([150, 300, 300], [3, 2, 1], 8),
+                                            ([32, 15, 15, 32, 15, 15], [4, 3, 6, 2, 1, 5], 4)])
+def test_plans_that_small_cells_cannot_beat_are_searched_once(pt, dims, perm, elem):
+    a = ((ctypes.c_int64 * len(dims))(*dims), (ctypes.c_int * len(perm))(*perm), len(dims), elem)
+    without, both = pt.pt_plan_ms(*a, 0, 9), pt.pt_plan_ms(*a, 1, 9)
+    assert 0 < both < 1.5 * without, (without, both)
