@@ -272,9 +272,11 @@ struct Tuning {
   int64_t min_groups = 1024;        // workgroups a single-launch pass spreads its footprints over
   int64_t whole = 1;                // whole-permutation passes (whole.hpp) where they fit
   // microseconds that a resident pass's workgroups wait for each other: they
-  // meet within microseconds, unless other work holds the chip (ms); what
-  // follows then takes milliseconds too
-  int64_t whole_patience = 100000;
+  // meet within microseconds, unless other work holds the chip; no longer than
+  // moving a region alone takes (0.1 to 34 ms).  Three processes at once, 4 s
+  // of calls of 16 to 64 MB: calls of up to 101-154 ms with 100 ms, 35-66 with
+  // 20, 57-68 with 5, 45 with ordinary passes only.
+  int64_t whole_patience = 20000;
   bool plain = true;   // every knob of the passes has its default value
   uint64_t epoch = 0;  // bumped on every change (plan caches key on it)
 };

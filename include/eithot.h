@@ -62,7 +62,9 @@ int eithot_transpose(void* dev, const int64_t* dims, const int* perm, int order,
  * own (within the same bound, counted by eithot_last_peak_extra_bytes of the
  * capturing call), which the graph owns: replays may come at any time and
  * beside any other call.  The memory is freed by the first transpose or
- * eithot_release after the graph and its executables are destroyed. */
+ * eithot_release after the graph and its executables are destroyed.  (An
+ * executable that hipGraphExecUpdate points at another graph does not keep
+ * that graph's memory: destroy the graph after it.) */
 int eithot_transpose_async(void* dev, const int64_t* dims, const int* perm, int order,
                            size_t elem_bytes, int n_sub, double alpha, void* stream);
 
@@ -96,7 +98,8 @@ int eithot_inplace_transpose(void* data, int source, int rank, const int* dim,
  * tuning value (64 MiB, which spares calls on small tensors from evicting
  * and re-uploading each other's tables).  0 when nothing is held.
  * Server pools and batch scratch belong to their handles and are not
- * counted. */
+ * counted, nor are the counters of resident passes (1.2 MB per device, held
+ * with the library's code). */
 size_t eithot_last_peak_extra_bytes(void);
 
 /* How the calling thread's last transpose ran: 0 the plan's passes, 1 or 2
@@ -261,7 +264,7 @@ int eithot_plan_segments(const int64_t* dims, const int* perm, int order, size_t
  *                    0: never).  Off while any knob of the passes differs
  *                    from its default; regions need a stream that sees the
  *                    whole chip and is not captured
- *   "whole_patience" microseconds (100000; 0 to 60000000) that the workgroups of
+ *   "whole_patience" microseconds (20000; 0 to 60000000) that the workgroups of
  *                    such a region wait for each other.  Where other work
  *                    keeps them apart for longer, the region is moved through
  *                    pinned host memory by one workgroup (1 to 64 MiB, as
@@ -309,7 +312,8 @@ int eithot_batch_add(eithot_batch* b, void* dev, const int64_t* dims, const int*
 int eithot_batch_build(eithot_batch* b, double alpha, int tune);
 /* Replays the batch on `stream` (NULL: null stream) and waits when sync. */
 int eithot_batch_run(eithot_batch* b, void* stream, int sync);
-/* Launch count per replay and the batch's scratch bytes. */
+/* Launch count per replay and the batch's scratch bytes (its launches' lists
+ * of tensors, blocks and counters come on top). */
 int eithot_batch_info(const eithot_batch* b, int* launches, int64_t* scratch_bytes,
                       int* graph_captured);
 void eithot_batch_destroy(eithot_batch* b);
