@@ -263,7 +263,10 @@ static bool sees_all_cus(int cus, hipStream_t stream) {
 bool Device::takes_whole_locked(const Plan& plan, hipStream_t stream) {
   if (!plan.whole) return false;
   if (plan.whole->mode == WHOLE_ORBIT) return true;
-  return sees_all_cus(prof.cus, stream) && whole_begin_locked(plan.whole->g.region, stream);
+  // the null stream's mask is the runtime's, which stays: asked for once
+  if (!stream && !null_sees_all) null_sees_all = sees_all_cus(prof.cus, nullptr) ? 1 : -1;
+  if (stream ? !sees_all_cus(prof.cus, stream) : null_sees_all < 0) return false;
+  return whole_begin_locked(plan.whole->g.region, stream);
 }
 
 bool Device::whole_room_locked(uint64_t region) {

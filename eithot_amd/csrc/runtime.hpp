@@ -42,6 +42,7 @@ struct Device {
   // under enqueue_mu.
   hipEvent_t whole_ready = nullptr;
   bool whole_elsewhere = false;      // the last one ran on a stream other than the null stream
+  int null_sees_all = 0;             // the null stream has every CU: 1, not: -1
   WholeCtl whole_ctl;
   // bytes at whole_ctl.room: a power of two, 1 to 64 MiB.  A smaller room
   // before it stays, for the passes in flight and the batches that name it.
