@@ -58,6 +58,8 @@ int eithot_transpose(void* dev, const int64_t* dims, const int* perm, int order,
  * Calls may come from several threads: the launches of calls that use the
  * arena or pass tables are enqueued one call at a time, and a call's first
  * pass waits (on the device) for the last pass of the previous arena user.
+ * Calls that run as one whole pass over regions (eithot_last_whole_pass 2)
+ * follow each other in the same way.
  * On a stream under capture the call's scratch and tables are memory of its
  * own (within the same bound, counted by eithot_last_peak_extra_bytes of the
  * capturing call), which the graph owns: replays may come at any time and
