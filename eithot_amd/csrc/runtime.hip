@@ -641,12 +641,12 @@ static int transpose_impl(void* dev, const int64_t* dims, const int* perm, int o
     if (!g_err.size()) fail(rc, "planning failed (%d)", rc);
     return rc;
   }
-  d->free_retired();
   if (stream_captured(stream))
     return transpose_captured(
         d, plan,
         [&](int* err) { return d->plan_for(dims, perm, order, elem, n_sub, alpha, err, false); },
         (char*)dev, stream);
+  d->free_retired();  // not inside a capture: it waits for the device
   {
     std::lock_guard<std::mutex> lk(d->enqueue_mu);
     const bool whole = d->takes_whole_locked(*plan, stream);

@@ -63,8 +63,8 @@ int eithot_transpose(void* dev, const int64_t* dims, const int* perm, int order,
  * On a stream under capture the call's scratch and tables are memory of its
  * own (within the same bound, counted by eithot_last_peak_extra_bytes of the
  * capturing call), which the graph owns: replays may come at any time and
- * beside any other call.  The memory is freed by the first transpose or
- * eithot_release after the graph and its executables are destroyed.  (An
+ * beside any other call.  The memory is freed by the first transpose that
+ * is not captured, or eithot_release, after the graph and its executables are destroyed.  (An
  * executable that hipGraphExecUpdate points at another graph does not keep
  * that graph's memory: destroy the graph after it.) */
 int eithot_transpose_async(void* dev, const int64_t* dims, const int* perm, int order,

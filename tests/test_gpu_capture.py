@@ -109,6 +109,25 @@ def test_graphs_give_their_memory_back(torch_cuda):
     assert torch.cuda.mem_get_info()[0] >= free + 32 * need
 
 
+def test_capture_after_a_graph_has_ended(torch_cuda):
+    # memory that an ended graph has let go of waits for a call outside the capture
+    torch = torch_cuda
+    x = Case(torch, CASES[0][0], CASES[0][1], 4, 14)
+    for mode in (THREAD_LOCAL, GLOBAL, RELAXED):
+        g = Graph(x.call, mode)
+        g.close()
+        torch.cuda.synchronize()
+        time.sleep(0.3)
+        g = Graph(x.call, mode)
+        for k in range(3):
+            x.buf.copy_(x.src)
+            torch.cuda.synchronize()
+            g.replay()
+            g.wait()
+            x.check(f"replay {k}")
+        g.close()
+
+
 def test_capture_mode_is_left_as_it_was(torch_cuda):
     # two calls in one capture, beside torch's own work
     torch = torch_cuda
